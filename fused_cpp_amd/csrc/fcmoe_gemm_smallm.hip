@@ -159,13 +159,14 @@ __device__ __forceinline__ void smallm_body(const SmallMArgs& p, int bx, int by)
     (issue(S, std::integral_constant<int, S>{}), ...);
   }(std::make_integer_sequence<int, D - 1>{});
 
-  auto body = [&](int t, auto slot_c) {
+  // Chunk t's fragments and MFMAs. The scheduling barrier keeps the MFMAs, and
+  // with them the waits for this wave's fragment reads, ahead of the next
+  // chunk's workgroup barrier: past that barrier the other waves' loads
+  // overwrite this stage (left free, the compiler moved the last rows' MFMAs
+  // and their waits behind it, and a read still queued then could return the
+  // next contents).
+  auto compute = [&](auto slot_c) {
     constexpr int slot = decltype(slot_c)::value;
-    // this wave's pair t has landed (pairs t+1 .. t+D-2 may not); after the
-    // barrier every wave's A stage t has, and no wave reads stage t-1 any more
-    sm_wait_vmcnt<OPS * (D - 2)>();
-    __builtin_amdgcn_s_barrier();
-    issue(t + D - 1, std::integral_constant<int, (slot + D - 1) % D>{});
     v4i af[FM];
 #pragma unroll
     for (int i = 0; i < FM; ++i) af[i] = *(const v4i*)(sa + slot * ABYTES + i * 1024 + frag);
@@ -176,19 +177,39 @@ __device__ __forceinline__ void smallm_body(const SmallMArgs& p, int bx, int by)
       else
         acc[i] = mfma(__builtin_bit_cast(v8bf, af[i]), __builtin_bit_cast(v8bf, bq[slot]), acc[i]);
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  // whole rings of D chunks, then the rest: no conditional step inside the
+  auto body = [&](int t, auto slot_c) {
+    constexpr int slot = decltype(slot_c)::value;
+    // this wave's pair t has landed (pairs t+1 .. t+D-2 may not); after the
+    // barrier every wave's A stage t has, and no wave reads stage t-1 any more
+    sm_wait_vmcnt<OPS * (D - 2)>();
+    __builtin_amdgcn_s_barrier();
+    issue(t + D - 1, std::integral_constant<int, (slot + D - 1) % D>{});
+    compute(slot_c);
+  };
+  // Whole rings of D chunks, then the rest: no conditional step inside the
   // loop, so the compiler's wait counts at the loop header match the steady
-  // state (a conditional step made it wait for all but the newest pair)
+  // state (a conditional step made it wait for all but the newest pair). The
+  // rest's pairs (fewer than D) are all in flight when the loop ends, so its
+  // steps issue none and wait for one pair fewer each: a step that issued
+  // pairs nobody reads lost their weight loads to the compiler, and with them
+  // the count its wait assumed.
   int t0 = 0;
   for (; t0 + D <= nch; t0 += D) {
     [&]<int... S>(std::integer_sequence<int, S...>) {
       (body(t0 + S, std::integral_constant<int, S>{}), ...);
     }(std::make_integer_sequence<int, D>{});
   }
+  auto rest = [&](auto slot_c) {
+    constexpr int slot = decltype(slot_c)::value;
+    sm_wait_vmcnt<OPS * (D - 2 - slot)>();
+    __builtin_amdgcn_s_barrier();
+    compute(slot_c);
+  };
   [&]<int... S>(std::integer_sequence<int, S...>) {
-    ((t0 + S < nch ? body(t0 + S, std::integral_constant<int, S>{}) : void()), ...);
-  }(std::make_integer_sequence<int, D>{});
+    ((t0 + S < nch ? rest(std::integral_constant<int, S>{}) : void()), ...);
+  }(std::make_integer_sequence<int, D - 1>{});
   sm_wait_vmcnt<0>();
 
   if (!tv) return;

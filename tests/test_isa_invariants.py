@@ -114,6 +114,45 @@ def _vgprs(asm: str) -> dict[str, int]:
     return dict(zip(names, counts))
 
 
+@pytest.fixture(scope="module")
+def smallm_asm(tmp_path_factory) -> str:
+    hipcc = ROCM / "bin" / "hipcc"
+    if not hipcc.exists():
+        pytest.skip("hipcc not available")
+    out = tmp_path_factory.mktemp("isa") / "fcmoe_gemm_smallm.s"
+    proc = subprocess.run([str(hipcc), *HIP_FLAGS, "--cuda-device-only", "-S", str(CSRC / "fcmoe_gemm_smallm.hip"),
+                           "-o", str(out)], capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+    return out.read_text()
+
+
+def test_small_m_stage_reads_end_before_the_barrier(smallm_asm):
+    """The small-M kernel's stages are refilled right after the workgroup
+    barrier, so no fragment read may still be queued when a wave reaches it:
+    a wait for every LDS read lies between the last read and the barrier. And
+    the steps after the K loop issue no loads, so that their vmcnt counts are
+    the ones the source computes."""
+    kernels = re.findall(r"^(_Z\w*smallm_(?:pair_)?kernel\w*):(.*?)\.Lfunc_end", smallm_asm, re.M | re.S)
+    assert len(kernels) >= 15
+    for name, text in kernels:
+        body = text.splitlines()
+        pending = False
+        barriers = 0
+        for line in body:
+            op = line.strip()
+            if op.startswith("ds_read"):
+                pending = True
+            elif op.startswith("s_waitcnt") and "lgkmcnt(0)" in op:
+                pending = False
+            elif op.startswith("s_barrier"):
+                barriers += 1
+                assert not pending, (name, barriers)
+        assert barriers >= 15, name
+        last_loop_load = max(i for i, line in enumerate(body) if "buffer_load" in line)
+        later = [i for i, line in enumerate(body) if line.strip().startswith("s_barrier") and i > last_loop_load]
+        assert len(later) >= 7, (name, len(later))
+
+
 def test_mixed_plan_register_budget(lds_asm, tmp_path):
     """The mixed prefill plan relies on one workgroup of the persistent MFMA
     kernel (two waves per SIMD) and one of the 16-row streaming kernel (one
