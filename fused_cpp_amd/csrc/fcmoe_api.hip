@@ -256,6 +256,11 @@ struct SideStreams {
   hipEvent_t join[kNumClasses] = {};
 };
 constexpr int kMaxDevices = 64;
+// Side streams a stage forks at most: with the caller's stream one per
+// hardware queue of a process (4). A fifth stream shares a queue with another
+// one, and its launch starts only when that one's is done: the W8A16 128-row
+// class queued behind the 192-row class (DSv3, T=4096: W13 1.36 + 1.07 ms).
+constexpr int kSides = 3;
 thread_local SideStreams t_side[kMaxDevices];
 
 int side_streams(SideStreams** out) {
@@ -332,13 +337,20 @@ int run_classes(const TileClasses& tc, hipStream_t stream, F&& gemm, bool serial
   if (rc) return rc;
   if (hipEventRecord(ss->fork, stream) != hipSuccess) return fail(FCMOE_EDEVICE, "hipEventRecord failed");
   if ((rc = gemm(tc.n - 1, stream))) return rc;
-  for (int c = tc.n - 2; c >= 0; --c) {
-    if ((rc = fork_wait(ss->s[c], ss->fork, stream, stream))) return rc;
-    if ((rc = gemm(c, ss->s[c]))) return rc;
-    if (hipEventRecord(ss->join[c], ss->s[c]) != hipSuccess) return fail(FCMOE_EDEVICE, "hipEventRecord failed");
+  // side stream k takes class n - 2 - k; the last one also the smaller
+  // classes, whose launches have little work
+  const int sides = tc.n - 1 < kSides ? tc.n - 1 : kSides;
+  for (int k = 0; k < sides; ++k) {
+    hipStream_t s = ss->s[k];
+    if ((rc = fork_wait(s, ss->fork, stream, stream))) return rc;
+    for (int c = tc.n - 2 - k; c >= 0; --c) {
+      if ((rc = gemm(c, s))) return rc;
+      if (k < sides - 1) break;
+    }
+    if (hipEventRecord(ss->join[k], s) != hipSuccess) return fail(FCMOE_EDEVICE, "hipEventRecord failed");
   }
-  for (int c = tc.n - 2; c >= 0; --c)
-    if ((rc = fork_wait(stream, ss->join[c], ss->s[c], stream))) return rc;
+  for (int k = 0; k < sides; ++k)
+    if ((rc = fork_wait(stream, ss->join[k], ss->s[k], stream))) return rc;
   return FCMOE_OK;
 }
 
@@ -586,18 +598,20 @@ int run_w8a8_stage(const TileClasses& tc, const RouteBuffers& rb, int epi, const
     // the streaming ones arrive), the rest on three side streams; the plan
     // not taken exits at once, beside the one that runs. The device has 4
     // hardware queues, so launches are paired on streams such that at most
-    // one of a pair has much work under either plan: the 16-row streaming
-    // launch, then the classic 16-row class (the mixed plan runs the first,
-    // the classic plan the second); the classic 256-row class (it exits when
-    // the persistent launch takes it), then the 128-row class; the 192-row
-    // class alone. (With a stream per launch, C4's 128-row launch queued
-    // behind the 192-row one on a shared hardware queue.)
+    // one of a pair has work under either plan: the persistent launch, then
+    // the classic 256-row class (which exits when the persistent launch takes
+    // it); the 16-row streaming launch, then the classic 16-row class (the
+    // mixed plan runs the first, the classic plan the second); the 128-row
+    // class alone; the 192-row class alone. The MFMA-bound 256-row class and
+    // the HBM-bound 128-row one then overlap whenever both have work: behind
+    // the 256-row class on one stream, the 128-row class of a Zipf-routed
+    // DSv3 layer at T=4096 started after it (W13 0.93 + 0.95 ms).
     SideStreams* ss = nullptr;
     if ((rc = side_streams(&ss))) return rc;
     if (hipEventRecord(ss->fork, stream) != hipSuccess) return fail(FCMOE_EDEVICE, "hipEventRecord failed");
     if ((rc = gemm_launch(epi, 256, pm, big_bound, stream))) return rc;
     const bool with_classic = gate.plan_min > 0;  // forced mixed plan: no classic launches
-    constexpr int kSides = 3;
+    if (with_classic && (rc = classic(3, stream))) return rc;
     for (int k = 0; k < kSides; ++k) {
       hipStream_t s = ss->s[k];
       if ((rc = fork_wait(s, ss->fork, stream, stream))) return rc;
@@ -606,8 +620,7 @@ int run_w8a8_stage(const TileClasses& tc, const RouteBuffers& rb, int epi, const
         if ((rc = gemm_launch(epi, 16, ps, tc.bound[0], s))) return rc;
         if (with_classic && (rc = classic(0, s))) return rc;
       } else if (with_classic) {
-        if ((rc = classic(k == 1 ? 3 : 2, s))) return rc;
-        if (k == 1 && (rc = classic(1, s))) return rc;
+        if ((rc = classic(k, s))) return rc;
       }
       if (hipEventRecord(ss->join[k], s) != hipSuccess) return fail(FCMOE_EDEVICE, "hipEventRecord failed");
     }
