@@ -661,9 +661,15 @@ __device__ __forceinline__ void lds_gemm_body(const GemmParams& p, int n_blocks,
     (void)tile_of(wn, j, &v);
     wave_live = wave_live || v;
   }
-  // Persistent launches also take experts of fewer rows than the tile: a
-  // wave whose row fragments all lie past the expert's rows skips its MFMAs.
-  if constexpr (PERSIST) wave_live = wave_live && wm * FM * 16 < rows;
+  // A wave whose row fragments all lie past the tile's rows skips its reads
+  // and MFMAs, and a wave with some of them past the rows skips those.
+  // Persistent launches take experts of fewer rows than the tile, and the
+  // 128-row class holds experts of 17 rows up (a Zipf-routed DSv3 layer at
+  // T=4096: 3.18 -> 3.15 ms). The wider tiles' rows mostly fill them, and the
+  // test per fragment costs them more (an i8gemm of 4096 full rows 0.439 ->
+  // 0.457 ms; the 192-row tile spills).
+  constexpr bool SKIP = PERSIST || BM == 128;
+  if constexpr (SKIP) wave_live = wave_live && wm * FM * 16 < rows;
   // row fragments of this wave that hold rows of the expert (the rest are clamped re-reads of its last row)
   const int live_frags = __builtin_amdgcn_readfirstlane((rows - wm * FM * 16 + 15) / 16);
 
@@ -758,9 +764,10 @@ __device__ __forceinline__ void lds_gemm_body(const GemmParams& p, int n_blocks,
     __builtin_amdgcn_sched_group_barrier(0x100, FN + 2, 0);  // the FN + 2 leading LDS reads
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
+      // row fragments past the tile's rows: no further reads or MFMAs
+      if constexpr (SKIP)
+        if (i >= live_frags) break;
       if (i + 2 < FM) af[(i + 2) % 3] = *(const v4i*)(sta + (i + 2) * A_FRAG);
-      // persistent launches: row fragments past the expert's rows skip their MFMAs
-      if (PERSIST && i >= live_frags) continue;
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         if constexpr (I8) {
