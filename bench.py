@@ -179,8 +179,10 @@ def expert_counts(cfg, ids):
     return counts
 
 
-CLASS_BM_PREFILL = (16, 128, 192, 256)  # W8A8 / BF16 prefill tile classes
-CLASS_BM_W8 = (16, 32, 128, 192, 256)  # W8A16 tile classes
+# Tile classes of the benchmark's prefill layers (over 4 GB of weights, more than 96 rows per expert
+# on average); smaller calls take one class of fcmoe_api.hip's select_classes.
+CLASS_BM_PREFILL = (16, 128, 192, 256)  # W8A8
+CLASS_BM_W8 = (128, 192, 256)  # W8A16 tile classes
 
 
 def class_of(c: int, decode: bool, kind: str = "w8a8") -> int:

@@ -4,6 +4,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -25,13 +26,6 @@ thread_local std::string g_error;
 constexpr int kClassBM[] = {16, 32, 64, 128, 192, 256};
 constexpr int kI8ClassBM[] = {256};  // i8gemm above kSmallMRows rows
 constexpr int kNumClasses = 6;
-// Decode: when an expert averages at most this many routed rows, everything
-// (the shared expert too, in several 16-row tiles) runs in the single BM=16
-// class: one launch per GEMM stage, no empty class launches, and weight
-// streaming is the only cost (a multi-tile expert re-reads its weights from
-// L2 / Infinity Cache, not HBM, since its tiles run side by side).
-constexpr int kDecodeRowsPerExpert = 8;
-
 // Stage-timing slot of a class: the index of its BM in kClassBM, so a stage
 // is named by its tile rows whatever class set the forward uses.
 int class_slot(int bm) {
@@ -40,35 +34,101 @@ int class_slot(int bm) {
   return kNumClasses - 1;
 }
 
-// Prefill (W8A8 and BF16): experts of 17-128 rows take the LDS-staged
-// 128-row tile rather than the register-ring 32/64-row tiles. Their weights
-// are read once either way, and the staged tile streams them faster with one
-// class launch fewer per stage. Measured on the DSv3 W8A8 layer: T=1024
-// 2.41 -> 2.17 ms, T=2048 2.63 -> 2.36, C3 3.27 -> 3.19, C4 4.68 -> 4.66;
-// BF16 at T=512 / 4096 unchanged. Keeping either the 32- or the 64-row class
-// made C3 slower (3.32 / 3.37 ms).
+// The tile classes of a forward, chosen from what the host knows: the average
+// rows per expert r = routes / experts, the bytes of all its experts' weights
+// and the operations. One class is one launch per GEMM stage on the caller's
+// stream; several classes are several launches on forked streams (about 4 us
+// of host time each and 20-40 us of fork and join per forward). us per forward
+// on MI355X, H = 7168, F = 2048, 256 experts + 1 shared, top-8 ("DSv3"), H =
+// 4096, F = 512, 20 experts + 1 shared, top-6 ("TP"), H = 1024, F = 512, 8
+// experts, top-2 ("8x512"):
+//   * 16-row tiles (register-ring kernel, weights streamed once per 16 rows)
+//     while experts see a row or two: DSv3 W8A8 T=64 (r = 2.2) 1490 against
+//     1510 on 64-row tiles, T=128 (r = 4.5) 1706 against 1704. BF16 and W8A16
+//     move to 64 rows at r = 2 (128 experts, r = 2.2: BF16 1537 -> 1508, DSv3
+//     W8A16 T=64 1508 -> 1490; 384 experts BF16 T=70, r = 1.6, 3991 against
+//     4142), and so does a layer whose W2 is a short K over
+//     many experts, where the 16-row kernel's workgroups are all set-up (DSv3
+//     with F = 256 T=16 161 -> 114, T=100 389 -> 278; the few workgroups of TP
+//     at T=2 stay, 30 against 37). Layers that fit an L2 stay up to r = 32
+//     (8x512 T=100 27 against 31).
+//   * 64-row tiles (fcmoe_gemm_mid.hip) from there to r = 48, and beyond it
+//     while the layer's operations are few: what a larger tile would save in
+//     weight re-reads is less than what its longer K walk on a few dozen
+//     workgroups costs. TP W8A8 T=200 180 -> 66, T=1000 244 -> 146; BF16 T=200
+//     253 -> 94, T=1000 322 -> 225; W8A16 T=400 246 -> 88 (the start's side:
+//     class launches on forked streams). The operations bound: TP BF16 T=1000
+//     (88 GFLOP) 225 against 257 on 128 rows, T=2047 (180) 422 against 319;
+//     one BF16 expert at 1000 rows (88) 246 against 288, at 2000 (180) 478
+//     against 332; 8 DSv3 W8A8 experts at T=256 (203 GOP) 298 against 181.
+//   * 128-row tiles above; 256-row ones when experts hold many tiles of either
+//     (r > 1000: TP W8A8 T=4000 363 against 401, BF16 569 against 599).
+//   * Layers of more than kBigWeights: 64 rows up to r = 10 (W8A8; T=256 1871 ->
+//     1808), 16 (BF16; 128 experts T=128 1840 -> 1751) or 24 (W8A16; T=512 2119
+//     -> 1923); one 128-row class up to r = 48 (W8A8 T=1024 2078 -> 2030,
+//     Zipf-routed 2476 -> 2110); above that {128, 192, 256} side by side (BF16
+//     128 experts T=1024 2130 -> 2096, W8A16 T=2048 2656 -> 2622, T=4096 4100
+//     -> 4051). W8A8 above r = 96 keeps the launch plans of run_w8a8_stage.
+enum Family { kW8A8, kBf16, kW8A16 };
+constexpr int64_t kBigWeights = 4ll << 30;
+// Layers of more weight bytes than this do not stay in the Infinity Cache (256
+// MB): 64-row tiles that read an expert once (r <= 48) load them nontemporal
+// (DSv3 T=64 1623 -> 1510, one 8-expert layer of 132 MB 50 -> 55).
+constexpr int64_t kCachedWeights = 300ll << 20;
+
 constexpr int kPrefillClassBM[] = {16, 128, 192, 256};
 constexpr int kNumPrefillClasses = 4;
 
-// Few rows in all (a dense MLP or i8gemm at decode batch sizes, a small MoE
-// batch): the 16-row class, whose one- or eight-wave workgroups spread the
-// weight stream over every CU. A larger class would give one workgroup per
-// channel block and row tile, e.g. 8 for the DSv3 shared MLP at 64 rows on
-// the 128-row tile; the 16-row tiles of one expert re-read its weights, which
-// the tiles running side by side find in L2 / Infinity Cache.
-// FCMOE_SMALL_ROWS overrides the bound (read on every call).
+struct MoeShape {
+  Family family;
+  int64_t routes, experts, hidden, inter;
+  int64_t elem() const { return family == kBf16 ? 2 : 1; }
+  int64_t weight_bytes() const { return 3 * hidden * inter * elem() * experts; }
+  bool few_rows(int64_t per_expert) const { return routes <= per_expert * experts; }
+};
+
+// FCMOE_SMALL_ROWS: routes up to which a forward runs on 16-row tiles whatever
+// its shape (default 64; read on every call).
 int64_t small_rows() {
   const char* v = getenv("FCMOE_SMALL_ROWS");
   return v && v[0] ? atoll(v) : 64;
 }
 
-bool decode_rows(int64_t routes, int64_t experts) {
-  return routes <= kDecodeRowsPerExpert * experts || routes <= small_rows();
-}
+bool weights_once(const MoeShape& m) { return m.few_rows(48) && m.weight_bytes() > kCachedWeights; }
 
-TileClasses select_classes(int64_t routes, int64_t experts) {
-  if (decode_rows(routes, experts)) return make_tile_classes(kClassBM, 1, routes, experts);
-  return make_tile_classes(kPrefillClassBM, kNumPrefillClasses, routes, experts);
+// FCMOE_TILE_CLASSES (tile rows in rising order, "128,192,256"): this class set
+// instead of the chosen one, so that tests and measurements reach every tile
+// at any shape; an unknown size is refused by its launch. Read on every call.
+// lds: the tiles above 32 rows can address A and one expert's weights (W8A16
+// has no other kernel for them).
+TileClasses select_classes(const MoeShape& m, bool lds = true) {
+  auto set = [&](std::initializer_list<int> bms) {
+    return make_tile_classes(bms.begin(), (int)bms.size(), m.routes, m.experts);
+  };
+  if (const char* v = getenv("FCMOE_TILE_CLASSES"); v && v[0] && lds) {
+    int bms[kMaxClasses], n = 0;
+    for (char* end; n < kMaxClasses && *v; v = *end ? end + 1 : end) bms[n++] = (int)strtol(v, &end, 10);
+    return make_tile_classes(bms, n, m.routes, m.experts);
+  }
+  const bool tiny = m.routes <= small_rows();
+  if (m.family == kW8A16 && !lds) return tiny || m.few_rows(8) ? set({16}) : set({16, 32});
+  const bool big = m.weight_bytes() > kBigWeights;
+  // 16-row tiles of a short W2 (at most 8 chunks of K) over many experts
+  const bool short_w2 = m.inter * m.elem() <= 512 && m.routes > 64 && m.weight_bytes() > kCachedWeights;
+  const bool in_l2 = m.weight_bytes() <= 64ll << 20;
+  const bool one_row = m.few_rows(m.family == kW8A8 ? 4 : 2);
+  if (tiny || (one_row && !short_w2) || (in_l2 && m.few_rows(32))) return set({16});
+  const char* forced = getenv("FCMOE_PREFILL_MIXED_MIN_TILES");
+  if (m.family == kW8A8 && ((big && !m.few_rows(96)) || (forced && forced[0])))
+    return make_tile_classes(kPrefillClassBM, kNumPrefillClasses, m.routes, m.experts);
+  if (big) {
+    if (m.few_rows(m.family == kW8A8 ? 10 : m.family == kBf16 ? 16 : 24)) return set({64});
+    if (m.few_rows(48) && m.family != kW8A16) return set({128});
+    return set({128, 192, 256});
+  }
+  const int64_t gop = 6 * m.routes * m.hidden * m.inter / 1000000000;
+  if (m.few_rows(48) || gop <= (m.family == kW8A8 ? 90 : m.family == kBf16 ? 120 : 110)) return set({64});
+  return m.few_rows(1000) ? set({128}) : set({256});
 }
 
 struct W8A8Layout {
@@ -127,7 +187,7 @@ W8A8Layout w8a8_layout(const fcmoe_moe_args* a, Arena& ar) {
   L.routes = a->tokens * L.kt;
   L.hp = round_up(a->hidden, 64);
   L.ip = round_up(a->inter, 64);
-  L.tc = select_classes(L.routes, a->experts);
+  L.tc = select_classes({kW8A8, L.routes, a->experts, a->hidden, a->inter});
   route_take(ar, L.rb, L.routes, a->experts, L.tc);
   L.xq = ar.take<int8_t>(a->tokens * L.hp);
   L.xs = ar.take<float>(a->tokens);
@@ -141,10 +201,6 @@ W8A8Layout w8a8_layout(const fcmoe_moe_args* a, Arena& ar) {
 
 // BF16 and W8A16 share this layout. K is padded to the GEMM's K chunk: 32
 // bf16 elements (64 bytes) for bf16 weights, 64 elements for int8 weights.
-// W8A16 tile classes: 16 / 32 rows on the direct-A kernel, 128 / 192 / 256
-// rows on the LDS-staged kernel (no 64-row W8A16 tile). The 192-row tile
-// takes experts of 129-192 rows off the 256-row one, which ran them at half
-// its rows (DSv3 shape, T = 4096 uniform: 4.63 -> 4.17 ms).
 // A BF16 forward over one packed expert with at most 256 routes (the shared
 // MLP, or a one-expert MoE, at decode batch sizes) runs its two GEMMs on the
 // small-M kernel (fcmoe_gemm_smallm.hip): every weight byte read once, K split
@@ -154,8 +210,6 @@ bool smallm_mlp(const fcmoe_moe_args* a, int64_t routes, bool w8) {
   return !w8 && a->experts == 1 && routes >= 1 && routes <= kSmallMRows && a->activation != FCMOE_ACT_SWIGLUOAI;
 }
 
-constexpr int kClassBMW8[] = {16, 32, 128, 192, 256};
-constexpr int kNumClassesW8 = 5;
 Bf16Layout bf16_layout(const fcmoe_moe_args* a, Arena& ar, bool w8 = false) {
   Bf16Layout L;
   const int64_t kmul = w8 ? 64 : 32;
@@ -164,18 +218,13 @@ Bf16Layout bf16_layout(const fcmoe_moe_args* a, Arena& ar, bool w8 = false) {
   L.hp = round_up(a->hidden, kmul);
   L.ip = round_up(a->inter, kmul);
   L.gu_ld = 2 * round_up(a->inter, 16);
-  // W8A16's 128/256-row tiles run on the LDS-staged kernel, whose buffer
+  // W8A16's tiles above 32 rows run on LDS-staged kernels, whose buffer
   // offsets are 32-bit: A and one expert's packed weights must stay under
   // 2 GiB; beyond that the forward keeps to the 16/32-row tiles.
   const bool w8_lds = a->tokens * L.hp * 2 < kLdsMaxABytes && L.routes * L.ip * 2 < kLdsMaxABytes &&
                       fcmoe_packed_expert_bytes(1, 2 * a->inter, a->hidden, 2) < kLdsMaxABytes &&
                       fcmoe_packed_expert_bytes(1, a->hidden, a->inter, 1) < kLdsMaxABytes;
-  if (w8)
-    L.tc = make_tile_classes(kClassBMW8,
-                             decode_rows(L.routes, a->experts) ? 1 : (w8_lds ? kNumClassesW8 : 2),
-                             L.routes, a->experts);
-  else
-    L.tc = select_classes(L.routes, a->experts);
+  L.tc = select_classes({w8 ? kW8A16 : kBf16, L.routes, a->experts, a->hidden, a->inter}, w8_lds);
   route_take(ar, L.rb, L.routes, a->experts, L.tc);
   L.xpad = (a->hidden % kmul) ? ar.take<uint16_t>(a->tokens * L.hp) : nullptr;
   L.y = ar.take<uint16_t>(L.routes * L.ip);
@@ -748,6 +797,7 @@ int w8a8_run(const fcmoe_moe_args* a, char* ws_base, size_t ws_bytes, bool seria
   }
 
   GemmParams g13{};
+  g13.weights_once = weights_once({kW8A8, L.routes, a->experts, H, I});
   g13.a = L.xq;
   g13.lda = L.hp;
   g13.a_rows = a->tokens;
@@ -777,6 +827,7 @@ int w8a8_run(const fcmoe_moe_args* a, char* ws_base, size_t ws_bytes, bool seria
   }
 
   GemmParams g2{};
+  g2.weights_once = g13.weights_once;
   g2.a = L.q2;
   g2.a_rows = L.routes;
   g2.lda = L.ip;
@@ -971,6 +1022,7 @@ int bf16_family_forward(const fcmoe_moe_args* a, hipStream_t stream, bool w8) {
     if (kt == 1) return FCMOE_OK;
   } else {
   GemmParams g13{};
+  g13.weights_once = weights_once({w8 ? kW8A16 : kBf16, L.routes, a->experts, H, I});
   g13.a = xa;
   g13.lda = L.hp;
   g13.a_rows = a->tokens;
@@ -1004,6 +1056,7 @@ int bf16_family_forward(const fcmoe_moe_args* a, hipStream_t stream, bool w8) {
     if (rc) return rc;
   }
   GemmParams g2{};
+  g2.weights_once = g13.weights_once;
   g2.a = L.y;
   g2.lda = L.ip;
   g2.a_rows = L.routes;

@@ -415,8 +415,11 @@ int gemm_launch(int epi, int bm, const GemmParams& p, int64_t max_tiles, hipStre
   const bool a_int8 = epi == kEpiRawI32 || epi == kEpiW13SwigluI8 || epi == kEpiW2RouteI8 || epi == kEpiI8Gemm;
   const bool a_fits = (p.a_rows <= 0 || p.a_rows * p.lda * (a_int8 ? 1 : 2) < kLdsMaxABytes) &&
                       p.w_expert_bytes < kLdsMaxABytes;  // one expert's weights: one buffer resource too
-  if (bm >= 128 && epi_w8(epi) && !a_fits)
+  if (bm >= 64 && epi_w8(epi) && !a_fits)
     return fail(FCMOE_EINVAL, "W8A16 LDS tiles need A and each expert's weights under 2 GiB");
+  // 64-row tiles of the forwards' own epilogues (the raw sums and the i8gemm keep the register-ring tile)
+  if (bm == 64 && a_fits && (use_lds || epi_w8(epi)) && epi != kEpiRawI32 && epi != kEpiI8Gemm)
+    return gemm_mid_launch(epi, p, max_tiles, stream);
   if (bm >= 128 && a_fits && (use_lds || epi_w8(epi))) return gemm_lds_launch(epi, bm, p, max_tiles, stream);
   if (epi == kEpiW13ActW8) return launch_bm_w8<kEpiW13ActW8>(bm, p, max_tiles, stream);
   if (epi == kEpiW2RouteW8) return launch_bm_w8<kEpiW2RouteW8>(bm, p, max_tiles, stream);

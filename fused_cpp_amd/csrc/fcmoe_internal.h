@@ -182,6 +182,9 @@ struct GemmParams {
   int64_t k_total;
   int32_t* split_out;
   int64_t split_rows;
+  // 64-row tiles: nonzero when the launch's experts mostly have one row tile
+  // and their weights exceed the caches: they are loaded nontemporal.
+  int weights_once;
 };
 
 // Whether a launch's plan gate lets it run (device side).
@@ -270,6 +273,8 @@ int smallm_bf16_launch(const SmallMBf16& q, hipStream_t stream);
 // LDS-staged kernel for bm in {128, 192, 256} (fcmoe_gemm_lds.hip); gemm_launch
 // dispatches to it unless FCMOE_GEMM_LDS=0.
 int gemm_lds_launch(int epi, int bm, const GemmParams& p, int64_t max_tiles, hipStream_t stream);
+// 64-row tiles (fcmoe_gemm_mid.hip), for the MoE forwards' epilogues.
+int gemm_mid_launch(int epi, const GemmParams& p, int64_t max_tiles, hipStream_t stream);
 // A bytes the LDS-staged kernel can address (32-bit buffer offsets).
 constexpr int64_t kLdsMaxABytes = 0x7ffffff0;
 

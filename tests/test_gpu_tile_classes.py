@@ -1,0 +1,87 @@
+"""Every tile class of the MoE forwards at the edges of its tiles: experts of
+1, 15, 16, 17, 63, 64, 65, 128, 129 and 260 rows, K of fewer chunks than a ring,
+whole rings and a ring with a remainder, channel counts that leave the last
+block part empty. FCMOE_TILE_CLASSES picks the class set at sizes whose rule
+would take another. W8A8 is compared bit for bit with the oracle; BF16 and
+W8A16 against the fp32 reference on the same bf16 values.
+Reference semantics: csrc/moe/arm/i8mm_w8a8/kernels.cpp:463-694,
+csrc/moe/arm/common/fused_moe_bf16_tiled.cpp:6376-7218."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from tests import helpers as H  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+ROWS = (1, 15, 16, 17, 63, 64, 65, 128, 129, 260)
+# 3 / 6, 16 / 32 and 10 / 20 chunks of K in W13 (int8 / bf16); 1 to 8 / 2 to 16 in W2
+SHAPES = [(192, 48), (1024, 512), (640, 208)]
+
+
+def _ids(rng):
+    ids = np.repeat(np.arange(len(ROWS)), ROWS)
+    rng.shuffle(ids)
+    return ids[:, None].astype(np.int64)
+
+
+@pytest.mark.parametrize("hd,f", SHAPES)
+@pytest.mark.parametrize("classes", ["16", "64", "128", "256", "128,192,256"])
+def test_w8a8_tile_edges_bit_exact(gpu, oracle_lib, monkeypatch, classes, hd, f):
+    ids = _ids(np.random.default_rng(hd + f))
+    x, _, w, q13, s13, q2, s2 = H.w8a8_case(hd * 3 + f, ids.shape[0], hd, f, len(ROWS), 1)
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
+    got = H.gpu_w8a8_forward(x, ids, w, q13, s13, q2, s2, gpu)
+    np.testing.assert_array_equal(got, oracle_lib.w8a8_forward(x, ids, w, q13, s13, q2, s2))
+
+
+@pytest.mark.parametrize("hd,f", SHAPES)
+@pytest.mark.parametrize("kind,classes", [("bf16", "64"), ("bf16", "128,192,256"), ("w8a16", "64"),
+                                          ("w8a16", "128,192,256")])
+def test_bf16_family_tile_edges(gpu, oracle_lib, monkeypatch, kind, classes, hd, f):
+    from fused_cpp_amd import moe
+
+    rng = np.random.default_rng(7 * hd + f)
+    E, ids = len(ROWS), _ids(rng)
+    x = H.bits_to_f32(H.bf16_bits(rng.standard_normal((ids.shape[0], hd)).astype(np.float32)))
+    b13 = H.bf16_bits((rng.standard_normal((E, 2 * f, hd)) * 0.05).astype(np.float32))
+    b2 = H.bf16_bits((rng.standard_normal((E, hd, f)) * 0.05).astype(np.float32))
+    w = rng.uniform(0.2, 1.0, (ids.shape[0], 1)).astype(np.float32)
+    bf = lambda b: torch.from_numpy(b.view(np.int16)).to(gpu).view(torch.bfloat16)  # noqa: E731
+    if kind == "bf16":
+        packed, call = moe.prepare_fused_moe_bf16_tiled_weights(bf(b13), bf(b2), fuse_silu=True), moe.fused_moe_bf16_tiled
+        f13, f2 = H.bits_to_f32(b13), H.bits_to_f32(b2)
+    else:
+        (q13, s13), (q2, s2) = oracle_lib.quant_weight_rows(b13), oracle_lib.quant_weight_rows(b2)
+        packed = moe.prepare_fused_moe_w8a16_tiled_quantized_weights(*map(torch.from_numpy, (q13, s13, q2, s2)))
+        call = moe.fused_moe_w8a16_tiled
+        f13, f2 = q13.astype(np.float32) * s13[..., None], q2.astype(np.float32) * s2[..., None]
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
+    out = call(bf(H.bf16_bits(x)), packed, torch.from_numpy(w).to(gpu), torch.from_numpy(ids).to(gpu))
+    got = out.float().cpu().numpy().astype(np.float64)
+    ref = oracle_lib.bf16_moe_reference(x, f13, f2, w, ids, round_intermediate=True).astype(np.float64)
+    # fp32 sums in another order leave the intermediate y within a few 2^-24 of the reference's, so a
+    # value next to a rounding boundary may fall on bf16's other side: one ulp, at most 2^-7 |y|, times
+    # its W2 weight and the route's. The chance is ~1e-4 a value, so two of a row's F values at most.
+    # On top of the result's own rounding (half a bf16 ulp) and fp32 sums over F terms.
+    ymax = np.empty((ids.shape[0], 1))
+    for e in range(E):
+        sel = ids[:, 0] == e
+        gate, up = np.split(x[sel].astype(np.float64) @ f13[e].T.astype(np.float64), 2, axis=1)
+        ymax[sel, 0] = np.abs(gate / (1.0 + np.exp(-gate)) * up).max(1)
+    step = ymax * np.abs(f2).max() * w
+    bound = H.bf16_half_ulp(ref) + 2 * 2.0 ** -7 * step + f * 2.0 ** -24 * step
+    assert (np.abs(got - ref) <= bound).all(), float((np.abs(got - ref) / bound).max())
+
+
+def test_w8a8_weights_read_once_bit_exact(gpu, oracle_lib):
+    """Enough experts that the 64-row tiles load weights nontemporal (over 300 MB), a few rows each."""
+    T, hd, f, E, k = 150, 1024, 512, 220, 8
+    x, ids, w, q13, s13, q2, s2 = H.w8a8_case(5, T, hd, f, E, k)
+    got = H.gpu_w8a8_forward(x, ids, w, q13, s13, q2, s2, gpu)
+    tok = np.array([0, 1, 74, T - 1])
+    np.testing.assert_array_equal(got[tok], oracle_lib.w8a8_forward(x[tok], ids[tok], w[tok], q13, s13, q2, s2))
