@@ -8,13 +8,18 @@
 // the appended shared expert with weight 1.0 and the routed weights are scaled
 // by routed_scaling_factor (src/fused_cpp/moe/bf16_tiled.py:1007-1013).
 //
-// Three launches, all O(routes):
+// One launch up to kOneLaunchRoutes routes (route_all_kernel): every
+// 1024-route workgroup builds the whole histogram over experts from the ids
+// itself, taking a copy before its own routes, so that no workgroup waits for
+// another; workgroup 0 also writes the counts, offsets and tile lists (the
+// tokens-per-expert tile selector), and extra workgroups quantise the W8A8
+// token rows. Beyond, three launches of O(routes) work in all:
 //   1. count:   per 256-route chunk, an LDS histogram over experts (the
 //               W8A8 token rows are quantised by extra workgroups of this
 //               launch).
 //   2. scan:    one block: per-expert exclusive scan over chunks, exclusive
 //               scan over experts (offsets), and the per-tile-class work lists
-//               for the grouped GEMMs (the tokens-per-expert tile selector).
+//               for the grouped GEMMs.
 //   3. scatter: per chunk, the in-chunk rank of each route among earlier
 //               routes of the same expert gives its stable sorted position.
 #include <utility>
@@ -29,7 +34,7 @@ namespace {
 
 constexpr int kScanThreads = 1024;
 constexpr int kMaxExperts = 1024;
-static_assert(kMaxExperts == kScanThreads, "the single-workgroup route kernel gives each expert a thread");
+static_assert(kMaxExperts == kScanThreads, "the one-launch route kernel gives each expert a thread");
 
 struct RouteArgs {
   const void* ids;
@@ -304,11 +309,6 @@ __global__ __launch_bounds__(kRouteChunk) void route_scatter_kernel(RouteArgs a,
   route_pos[r] = pos;
 }
 
-// Decode-sized routing (routes <= kScanThreads) in one workgroup, one route
-// per thread: LDS histogram, the expert scan and tile lists, then the stable
-// scatter, where a route's rank is the number of earlier routes of its expert
-// (a scan of the LDS expert list, four entries per read). Produces exactly
-// the outputs of the count / scan / scatter kernels.
 struct RouteOut {
   int32_t* counts;
   int32_t* offsets;
@@ -322,106 +322,137 @@ struct RouteOut {
   int32_t* queues;
 };
 
-__device__ __forceinline__ void route_small_body(const RouteArgs& a, int routes, const ClassArgs& cls,
-                                                 const RouteOut& o) {
-  int32_t* counts = o.counts;
-  int32_t* offsets = o.offsets;
-  int32_t* tiles = o.tiles;
-  int32_t* tile_count = o.tile_count;
-  int32_t* sorted_routes = o.sorted_routes;
-  int32_t* row_token = o.row_token;
-  int32_t* route_pos = o.route_pos;
-  float* route_weight = o.route_weight;
-  int32_t* invalid = o.invalid;
+// One-launch routing. Workgroup c owns routes 1024 c .. 1024 c + 1023 and counts
+// every route's expert into an LDS histogram: first the routes before its own
+// (hist is then each expert's routes in earlier chunks), then its own and the
+// later ones (hist is the expert's count, whose exclusive scan gives the
+// offsets). The redundant counting costs routes / 1024 id loads and LDS atomics
+// a thread, L2 hits all but the first; what it saves is two launches, each of
+// which waits for the one before. A route's rank among its wave's routes of the
+// same expert comes from ballots over the id's bits, the earlier waves' counts
+// from wcnt. DSv3 W8A8, route + row quantisation, MI355X: T=333 27 -> 8.5 us,
+// T=4096 47 -> 36, T=8192 E=384 73 -> 65; 64 tokens 11.8 -> 6.4 (there
+// one workgroup ranked each route against all earlier ones).
+constexpr int kOneLaunchRoutes = 1 << 18;
+constexpr int kRouteWaves = kScanThreads / kWave;
+constexpr int kIdBatch = 8;  // ids a thread has in flight
+
+// route_expert in 32 bits (the division is most of a counted id's work)
+__device__ __forceinline__ int route_expert32(const RouteArgs& a, uint32_t r, bool* valid) {
+  const uint32_t t = r / (uint32_t)a.kt, s = r - t * (uint32_t)a.kt;
+  if (s >= (uint32_t)a.top_k) return a.shared_id;
+  const uint32_t idx = t * (uint32_t)a.top_k + s;
+  const int64_t e = a.ids_is_i64 ? ((const int64_t*)a.ids)[idx] : (int64_t)((const int32_t*)a.ids)[idx];
+  *valid = e >= 0 && e < a.valid_experts;
+  return *valid ? (int)e : -1;
+}
+
+__device__ __forceinline__ void route_all_body(const RouteArgs& a, int routes, const ClassArgs& cls,
+                                               const RouteOut& o) {
   __shared__ int32_t hist[kMaxExperts];
-  __shared__ __attribute__((aligned(16))) int32_t ex[kScanThreads];
+  __shared__ uint16_t wcnt[kRouteWaves * kMaxExperts];  // [wave][expert] routes of the wave
   __shared__ int32_t n_invalid;
-  const int tid = threadIdx.x;
-  hist[tid] = 0;  // kMaxExperts == kScanThreads
+  const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+  const int r0 = (int)blockIdx.x * kScanThreads;
+  hist[tid] = 0;
+  for (int i = tid; i < kRouteWaves * a.experts; i += kScanThreads) wcnt[i] = 0;
   if (tid == 0) n_invalid = 0;
+  __syncthreads();
+  int bad = 0;
+  // experts of the routes [begin, end) into hist, kIdBatch loads at a time
+  auto count = [&](int begin, int end) {
+    for (int r = begin + tid; r < end; r += kIdBatch * kScanThreads) {
+      int e[kIdBatch];
+#pragma unroll
+      for (int u = 0; u < kIdBatch; ++u) {
+        const int q = r + u * kScanThreads;
+        bool valid = true;
+        e[u] = q < end ? route_expert32(a, (uint32_t)q, &valid) : -1;
+        bad += valid ? 0 : 1;
+      }
+#pragma unroll
+      for (int u = 0; u < kIdBatch; ++u)
+        if (e[u] >= 0) atomicAdd(&hist[e[u]], 1);
+    }
+  };
+  count(0, r0);
+  const int r = r0 + tid;
   int e = -1;
-  if (tid < routes) {
-    bool valid;
-    e = route_expert(a, tid, &valid);
-    route_weight[tid] = route_weight_of(a, tid);
+  if (r < routes) {
+    bool valid = true;
+    e = route_expert32(a, (uint32_t)r, &valid);
+    o.route_weight[r] = route_weight_of(a, r);
+    bad += valid ? 0 : 1;
   }
-  ex[tid] = e;  // -1: invalid or past the last route
-  __syncthreads();
-  if (tid < routes) {
-    if (e >= 0)
-      atomicAdd(&hist[e], 1);
-    else
-      atomicAdd(&n_invalid, 1);
+  // lanes of the wave with this lane's expert
+  uint64_t same = __ballot(e >= 0);
+  for (int bit = 0; (1 << bit) < a.experts; ++bit) {
+    const bool one = (e >> bit) & 1;
+    const uint64_t ones = __ballot(one);
+    same &= one ? ones : ~ones;
   }
+  const int rank = __popcll(same & ((1ull << lane) - 1));
+  if (e >= 0 && rank == 0) wcnt[wave * a.experts + e] = (uint16_t)__popcll(same);
   __syncthreads();
-  if (tid == 0) store_count(invalid, n_invalid);  // the count is written, not accumulated
+  int before = rank;
+  if (e >= 0) {
+    before += hist[e];
+    for (int w = 0; w < wave; ++w) before += wcnt[w * a.experts + e];
+  }
+  __syncthreads();  // every thread has read the earlier chunks' counts
+  if (e >= 0) atomicAdd(&hist[e], 1);
+  count(r0 + kScanThreads, routes);
+  if (blockIdx.x == 0 && bad) atomicAdd(&n_invalid, bad);
+  __syncthreads();
+  if (blockIdx.x == 0 && tid == 0) store_count(o.invalid, n_invalid);  // the count is written, not accumulated
   const bool owner = tid < a.experts;
-  const int count = owner ? hist[tid] : 0;
+  const int total_e = owner ? hist[tid] : 0;
   int total;
-  const int off = block_exclusive_scan(count, &total);
-  if (owner) {
-    counts[tid] = count;
-    offsets[tid] = off;
-  }
-  if (tid == 0) offsets[a.experts] = total;
-  emit_tiles(count, tid, cls, tiles, tile_count);
-  __syncthreads();  // every thread has read its hist entry
-  if (owner) hist[tid] = off;
+  const int off = block_exclusive_scan(total_e, &total);
+  hist[tid] = off;
   __syncthreads();
-  if (tid >= routes) return;
-  if (e < 0) {
-    route_pos[tid] = -1;
-    return;
+  if (r < routes) {
+    if (e >= 0) {
+      const int pos = hist[e] + before;
+      o.sorted_routes[pos] = r;
+      o.row_token[pos] = r / a.kt;
+      o.route_pos[r] = pos;
+    } else {
+      o.route_pos[r] = -1;
+    }
   }
-  int rank = 0;
-  const int4* ex4 = (const int4*)ex;
-  int j = 0;
-  for (; j + 4 <= tid; j += 4) {
-    const int4 q = ex4[j / 4];
-    rank += (q.x == e) + (q.y == e) + (q.z == e) + (q.w == e);
+  if (blockIdx.x != 0) return;
+  if (owner) {
+    o.counts[tid] = total_e;
+    o.offsets[tid] = off;
   }
-  for (; j < tid; ++j) rank += ex[j] == e;
-  const int pos = hist[e] + rank;
-  sorted_routes[pos] = tid;
-  row_token[pos] = tid / a.kt;
-  route_pos[tid] = pos;
+  if (tid == 0) o.offsets[a.experts] = total;
+  emit_tiles(total_e, tid, cls, o.tiles, o.tile_count);
 }
 
-__global__ __launch_bounds__(kScanThreads) void route_small_kernel(RouteArgs a, int routes, ClassArgs cls,
-                                                                   RouteOut o) {
-  zero_queues(o.queues);
-  route_small_body(a, routes, cls, o);
-}
-
-// Small-batch front end in one launch: workgroup 0 builds the routes as
-// route_small_kernel; workgroup b >= 1 quantises token rows 4 (b - 1) ..
-// 4 (b - 1) + 3, kRowThreads threads per row (quant_row_wg). The two jobs
-// are independent (the token rows do not depend on the routing), so they
-// share a launch instead of running back to back.
+// The token rows do not depend on the routing: workgroups past the routing's
+// quantise kQuantRowsPerGroup of them each, kRowThreads threads per row
+// (quant_row_wg). CAP 0: no rows.
 constexpr int kQuantRowsPerGroup = kScanThreads / kRowThreads;
 
-// Workgroup b >= 1 of a shared launch: token rows 4 (b - 1) .. 4 (b - 1) + 3.
 template <int CAP>
-__device__ __forceinline__ void quant_row_group(const QuantRows& qr) {
-  __shared__ float wmax[kScanThreads / kWave];
-  const int g = threadIdx.x / kRowThreads;
-  const int64_t row = (int64_t)(blockIdx.x - 1) * kQuantRowsPerGroup + g;
-  quant_row_wg<CAP>(qr.x, qr.cols, qr.rounding, qr.q, qr.ldq, qr.scales, row, row < qr.rows,
-                    (int)threadIdx.x % kRowThreads, wmax + g * (kRowThreads / kWave));
-}
-
-template <int CAP>
-__global__ __launch_bounds__(kScanThreads) void route_quant_small_kernel(RouteArgs a, int routes, ClassArgs cls,
-                                                                         RouteOut o, QuantRows qr) {
-  if (blockIdx.x == 0) {
+__global__ __launch_bounds__(kScanThreads) void route_all_kernel(RouteArgs a, int routes, int chunks, ClassArgs cls,
+                                                                 RouteOut o, QuantRows qr) {
+  if (CAP == 0 || (int)blockIdx.x < chunks) {
     zero_queues(o.queues);
-    route_small_body(a, routes, cls, o);
+    route_all_body(a, routes, cls, o);
     return;
   }
-  quant_row_group<CAP>(qr);
+  if constexpr (CAP > 0) {
+    __shared__ float wmax[kScanThreads / kWave];
+    const int g = threadIdx.x / kRowThreads;
+    const int64_t row = ((int64_t)blockIdx.x - chunks) * kQuantRowsPerGroup + g;
+    quant_row_wg<CAP>(qr.x, qr.cols, qr.rounding, qr.q, qr.ldq, qr.scales, row, row < qr.rows,
+                      (int)threadIdx.x % kRowThreads, wmax + g * (kRowThreads / kWave));
+  }
 }
 
-// Larger routings: the token rows are quantised by extra workgroups of the
+// Beyond: the token rows are quantised by extra workgroups of the
 // count launch (one row per kRowThreads-thread workgroup), so the column scan,
 // a single latency-bound workgroup, runs with the memory system to itself
 // (beside the quantisation it took C4's route from ~40 to ~72 us).
@@ -539,19 +570,21 @@ int route_launch(const void* ids, int ids_is_i64, const float* topk_w, int64_t t
   const int64_t chunks = ceil_div(routes, kRouteChunk);
   int32_t* invalid = invalid_out ? invalid_out : rb.invalid;
   const ClassArgs ca = class_args(tc);
-  if (routes <= kScanThreads) {
+  if (routes <= kOneLaunchRoutes) {
     const RouteOut o{rb.counts,    rb.offsets,   rb.tiles,        rb.tile_count, rb.sorted_routes,
                      rb.row_token, rb.route_pos, rb.route_weight, invalid,      rb.queues};
+    const int wgs = (int)ceil_div(routes, kScanThreads);
     if (const int cap = quant_done ? quant_cap(quant) : 0) {
-      const dim3 grid((unsigned)(1 + ceil_div(quant->rows, kQuantRowsPerGroup))), block(kScanThreads);
+      const dim3 grid((unsigned)(wgs + ceil_div(quant->rows, kQuantRowsPerGroup))), block(kScanThreads);
       with_cap(cap, [&](auto c) {
-        hipLaunchKernelGGL(route_quant_small_kernel<decltype(c)::value>, grid, block, 0, stream, a, (int)routes, ca,
-                           o, *quant);
+        hipLaunchKernelGGL(route_all_kernel<decltype(c)::value>, grid, block, 0, stream, a, (int)routes, wgs, ca, o,
+                           *quant);
       });
       *quant_done = true;
       return check_launch("route_quant");
     }
-    hipLaunchKernelGGL(route_small_kernel, dim3(1), dim3(kScanThreads), 0, stream, a, (int)routes, ca, o);
+    hipLaunchKernelGGL(route_all_kernel<0>, dim3((unsigned)wgs), dim3(kScanThreads), 0, stream, a, (int)routes, wgs,
+                       ca, o, QuantRows{});
     return check_launch("route");
   }
   if (const int cap = quant_done ? quant_cap(quant) : 0) {
