@@ -73,10 +73,11 @@ struct SmallMArgs {
                                // build drops invalid ids, so fewer than m rows may exist
 };
 
-__device__ __forceinline__ void sm_store(const SmallMArgs& p, int row, int64_t ch, int32_t acc) {
+__device__ __forceinline__ void sm_store(const SmallMArgs& p, int row, int64_t ch, int32_t acc, float rscale,
+                                         float cscale, float cbias) {
   // write_scaled_output, csrc/i8gemm.cpp:148-164 (left to right)
-  float v = (float)acc * p.scale_row[row] * p.scale_col[ch];
-  if (p.bias) v = v + p.bias[ch];
+  float v = (float)acc * rscale * cscale;
+  if (p.bias) v = v + cbias;
   if (p.out_bf16)
     ((uint16_t*)p.out)[(int64_t)row * p.ldo + ch] = f32_to_bf16(v);
   else
@@ -91,10 +92,14 @@ __device__ __forceinline__ void smallm_body(const SmallMArgs& p, int bx, int by)
   constexpr int D = kSmDepth;
   constexpr int ABYTES = FM * 1024;  // 16 FM rows x 64 bytes
   constexpr int LA = (FM + kSmWaves - 1) / kSmWaves;  // A loads per wave and chunk
+  static_assert(FM * 16 <= kSmWaves * kWave, "one row scale per thread");
   static_assert(FM <= kSmWaves || FM % kSmWaves == 0, "the waves' A loads cover every row fragment once");
   constexpr int OPS = LA + 1;  // vector-memory ops per (A stage, weight chunk) pair
   typedef typename Acc<I8>::type AccT;
-  __shared__ __attribute__((aligned(1024))) uint8_t sa[D * ABYTES];
+  // One LDS object (a second one made the compiler drain the ring before its
+  // fragment reads): the A stages, then the rows' scales.
+  __shared__ __attribute__((aligned(1024))) uint8_t sa[D * ABYTES + FM * 16 * 4];
+  float* const srow = (float*)(sa + D * ABYTES);
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int64_t tile = (int64_t)bx * kSmWaves + wave;  // packed tile (group-major)
@@ -135,6 +140,23 @@ __device__ __forceinline__ void smallm_body(const SmallMArgs& p, int bx, int by)
   const int voff_b = lane * 16;
   const int frag = (lane % 16) * 64 + (((lane / 16) ^ ((lane % 16) >> 2)) * 16);
 
+  // The direct epilogue's scales are loaded ahead of the K loop, the rows' into
+  // LDS: a load left between the epilogue's stores, which it may alias as far
+  // as the compiler knows, waits for the store before it (16 round trips at 64
+  // rows; the i8gemm pair [24576 + 8192, 1536] there 18.7 -> 16.2 us).
+  const int64_t grp = tile / p.n_tiles;
+  const int64_t cin = (tile - grp * p.n_tiles) * 16 + lane % 16;
+  const int64_t ch = grp * p.n_half + cin;  // logical channel
+  // (branch-free, from clamped places: a load in a conditional block is waited
+  // for at the block's end, before the ring starts)
+  float cscale = 0.0f, cbias = 0.0f, rscale = 0.0f;
+  if constexpr (I8) {
+    const int64_t cc = tv && cin < p.n_half ? ch : 0;
+    cscale = p.scale_col[cc];
+    cbias = (p.bias ? p.bias : p.scale_col)[cc];
+    rscale = p.scale_row[(int)threadIdx.x < p.m ? (int)threadIdx.x : 0];
+  }
+
   v4i bq[D];
   AccT acc[FM];
 #pragma unroll
@@ -158,6 +180,9 @@ __device__ __forceinline__ void smallm_body(const SmallMArgs& p, int bx, int by)
   [&]<int... S>(std::integer_sequence<int, S...>) {
     (issue(S, std::integral_constant<int, S>{}), ...);
   }(std::make_integer_sequence<int, D - 1>{});
+  // the K loop's first barrier publishes the rows' scales
+  if constexpr (I8)
+    if (threadIdx.x < FM * 16) srow[threadIdx.x] = rscale;
 
   // Chunk t's fragments and MFMAs. The scheduling barrier keeps the MFMAs, and
   // with them the waits for this wave's fragment reads, ahead of the next
@@ -212,11 +237,7 @@ __device__ __forceinline__ void smallm_body(const SmallMArgs& p, int bx, int by)
   }(std::make_integer_sequence<int, D - 1>{});
   sm_wait_vmcnt<0>();
 
-  if (!tv) return;
-  const int64_t grp = tile / p.n_tiles;
-  const int64_t cin = (tile - grp * p.n_tiles) * 16 + lane % 16;
-  if (cin >= p.n_half) return;
-  const int64_t ch = grp * p.n_half + cin;  // logical channel
+  if (!tv || cin >= p.n_half) return;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -228,7 +249,7 @@ __device__ __forceinline__ void smallm_body(const SmallMArgs& p, int bx, int by)
         if (p.partial)
           ((int32_t*)p.partial)[e] = acc[i][q];
         else
-          sm_store(p, row, ch, acc[i][q]);
+          sm_store(p, row, ch, acc[i][q], srow[row], cscale, cbias);
       } else {
         ((float*)p.partial)[e] = acc[i][q];
       }
@@ -262,7 +283,9 @@ __global__ __launch_bounds__(256) void smallm_reduce_kernel(SmallMArgs p, int sp
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
     int32_t acc = 0;
     for (int s = 0; s < splits; ++s) acc += ((const int32_t*)p.partial)[(int64_t)s * total + e];
-    sm_store(p, (int)(e / p.n), e % p.n, acc);
+    const int row = (int)(e / p.n);
+    const int64_t ch = e % p.n;
+    sm_store(p, row, ch, acc, p.scale_row[row], p.scale_col[ch], p.bias ? p.bias[ch] : 0.0f);
   }
 }
 
