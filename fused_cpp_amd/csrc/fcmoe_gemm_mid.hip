@@ -54,7 +54,15 @@ __global__ __launch_bounds__(kMidWaves * kWave) void grouped_gemm_mid_kernel(Gem
   static_assert(LA * 1024 * kMidWaves == ABYTES, "the waves' A loads cover the stage");
   constexpr int OPS = LA + FN;  // vector-memory ops per chunk and wave
   typedef typename Acc<I8>::type AccT;
-  __shared__ __attribute__((aligned(1024))) uint8_t sa[D * ABYTES];
+  // One LDS object: the A stages, then the epilogue's per-row and per-channel
+  // values (a second one would cost the K loop its counted waits).
+  constexpr int NT = kMidWaves * FN;  // channel tiles per workgroup
+  static_assert(NT * 16 <= kMidWaves * kWave && BM <= kMidWaves * kWave, "one value per thread");
+  constexpr int THREADS = kMidWaves * kWave;
+  __shared__ __attribute__((aligned(1024))) uint8_t sa[D * ABYTES + 12 * THREADS];
+  float* const meta_rs = (float*)(sa + D * ABYTES);
+  int* const meta_orow = (int*)(sa + D * ABYTES + 4 * THREADS);
+  float* const meta_cs = (float*)(sa + D * ABYTES + 8 * THREADS);
 
   // The dispatcher deals workgroups to the XCDs round-robin; workgroup b runs
   // item b / 8 of a contiguous range owned by XCD b % 8, tiles last-first with
@@ -125,6 +133,30 @@ __global__ __launch_bounds__(kMidWaves * kWave) void grouped_gemm_mid_kernel(Gem
                       : (lane % 16) * 64 + (((lane / 16) ^ ((lane % 16) >> 2)) * 16);
   const int dhi = (frag ^ 16) - frag;  // W8A16: the row's second unit of the chunk's 16-byte weight piece
 
+  // ---- the epilogue's row scales, output rows and channel scales: loaded
+  // ahead of the ring (thread t: row t, channel slot t) and kept in LDS. Loaded
+  // by the epilogue, each fragment's would wait for the stores of the one
+  // before it, and W13's row scale is a dependent pair of loads (W8A8 TP rank
+  // T=200 60 -> 55 us, 8x512 T=1000 52 -> 39).
+  constexpr bool ROUTE = epi_route(EPI), COLS = epi_col_scale(EPI);
+  const int mt = (int)threadIdx.x;
+  const int mpos = pos0 + (mt < rows ? mt : rows - 1);
+  int m_row = mpos, m_orow = mpos;
+  float m_rs = 0.0f, m_cs = 0.0f;
+  if constexpr (EPI == kEpiW13SwigluI8) {
+    if (p.row_map) m_row = p.row_map[mpos];
+    m_rs = p.scale_row[m_row];
+  }
+  if constexpr (EPI == kEpiW2RouteI8) m_rs = p.scale_row[mpos];
+  if constexpr (ROUTE) m_orow = p.sorted_routes[mpos];
+  if constexpr (COLS) {
+    // slot t / 16: wave t / 16 / FN's tile (t / 16) % FN
+    const int sw = mt / 16 / FN, sj = (mt / 16) % FN;
+    const int64_t g = PAIR ? sj : 0;
+    const int64_t cin = (PAIR ? (int64_t)nb * kMidWaves + sw : ((int64_t)nb * kMidWaves + sw) * FN + sj) * 16 + mt % 16;
+    m_cs = p.scale_col[(int64_t)expert * p.n + g * p.n_half + (sw < kMidWaves && cin < p.n_half ? cin : 0)];
+  }
+
   v4i bq[D][FN];
   AccT acc[FM][FN];
 #pragma unroll
@@ -151,6 +183,13 @@ __global__ __launch_bounds__(kMidWaves * kWave) void grouped_gemm_mid_kernel(Gem
   [&]<int... S>(std::integer_sequence<int, S...>) {
     (issue(S, std::integral_constant<int, S>{}), ...);
   }(std::make_integer_sequence<int, D - 1>{});
+
+  // Published by the K loop's first barrier. Every thread writes its entry (the
+  // epilogue reads the first BM and 16 NT): in a conditional block the loads
+  // would be sunk into it, behind the ring, and drain it.
+  meta_rs[mt] = m_rs;
+  meta_orow[mt] = m_orow;
+  meta_cs[mt] = m_cs;
 
   // The closing scheduling barrier keeps the MFMAs, and with them the waits
   // for this wave's fragment reads, ahead of the next chunk's workgroup
@@ -211,7 +250,8 @@ __global__ __launch_bounds__(kMidWaves * kWave) void grouped_gemm_mid_kernel(Gem
   }(std::make_integer_sequence<int, D - 1>{});
   mid_wait_vmcnt<0>();
 
-  gemm_epilogue<I8, EPI, FM, FN>(p, acc, gtile, tvalid, 0, rows, pos0, expert, lane);
+  const EpiMeta meta{(lds_cfloat_ptr)meta_rs, (lds_cint_ptr)meta_orow, (lds_cfloat_ptr)meta_cs, wave * FN};
+  gemm_epilogue<I8, EPI, FM, FN, true>(p, acc, gtile, tvalid, 0, rows, pos0, expert, lane, meta);
 #endif
 }
 
