@@ -562,16 +562,21 @@ bool part_enabled() {
   return !(v && v[0] == '0');
 }
 
-// Decode batches of at most this many tokens (FCMOE_DECODE_TAIL_MAX_T; 0
-// turns both off) run requant, W2 and the merge as one launch (the tail), and
-// a one-token batch runs route, row quantisation and W13 as one (the head).
-// At one token the tail saves two launches (C2 shape: 0.082 -> 0.077 ms) and
-// the head one more (0.074 ms); at two the tokens' workgroups each stream the
-// shared expert's weights, and the tail is slower (0.133 -> 0.136 ms).
-constexpr int kDecodeTailMaxTokens = 1;
-int decode_tail_max_tokens() {
-  const char* v = getenv("FCMOE_DECODE_TAIL_MAX_T");
-  return v && v[0] ? atoi(v) : kDecodeTailMaxTokens;
+// Batches that run a layer as two launches: the head (route, W8A8 row
+// quantisation, W13) and the tail (requant, W2, merge). One token always: the
+// launches it replaces are 3-5 us each around the same weight stream (DSv3
+// W8A8 0.082 -> 0.074 ms). More tokens while their routes fit a wave (64) and
+// their own weight streams together, mostly L2 reads, stay under
+// kSmallBatchBytes: each route streams its expert for itself, so a layer whose
+// launches are most of its time gains (us: 8 experts of 512 x 1024 top-2 W8A8 T=8
+// 26 -> 16, BF16 T=32 22 -> 17; TP rank of H 4096, F 512, top-6 BF16 T=1 30 -> 21,
+// W8A16 T=2 44 -> 22, W8A8 T=4 33 -> 27), and one that is bound by its
+// weights loses (DSv3 W8A8 T=2 120 -> 124 us, T=4 215 -> 227).
+// FCMOE_DECODE_TAIL_MAX_T, when set, is the W8A8 batches' rule instead: at most
+// this many tokens (0: none) take the tail, and one-token ones the head.
+constexpr int64_t kSmallBatchBytes = 200ll << 20;
+bool small_batch(int64_t tokens, int64_t routes, int64_t hidden, int64_t inter, int64_t elem) {
+  return tokens == 1 || (routes <= kWave && routes * 3 * hidden * inter * elem <= kSmallBatchBytes);
 }
 
 // One W8A8 GEMM stage (epilogue epi, stage-timing base id stage0) over the
@@ -712,7 +717,10 @@ int w8a8_run(const fcmoe_moe_args* a, char* ws_base, size_t ws_bytes, bool seria
   // the fused tail's whole launch domain (decode_tail_launch refuses anything
   // else), so that a larger FCMOE_DECODE_TAIL_MAX_T falls back to the unfused
   // launches instead of failing
-  const bool tail = a->tokens <= decode_tail_max_tokens() && a->tokens <= 65535 && L.kt <= kDecodeTailSlots &&
+  const char* max_t = getenv("FCMOE_DECODE_TAIL_MAX_T");
+  const bool by_env = max_t && max_t[0];
+  const bool small = small_batch(a->tokens, L.routes, H, I, 1);
+  const bool tail = (by_env ? a->tokens <= atoi(max_t) : small) && a->tokens <= 65535 && L.kt <= kDecodeTailSlots &&
                     parts <= 2 * kWave && H > 0;
   auto decode_tail = [&]() {
     // requant + W2 + merge in one launch (timed as the W2 16-row stage)
@@ -743,10 +751,11 @@ int w8a8_run(const fcmoe_moe_args* a, char* ws_base, size_t ws_bytes, bool seria
     Stage st(FCMOE_STAGE_W2_CLASS0 + class_slot(16), stream);
     return decode_tail_launch(d, stream);
   };
-  if (tail && a->tokens == 1 && L.hp <= kDecodeHeadMaxK && ceil_div(H / 8, 64) <= 16) {
-    // one token: route + row quantisation + W13 in one launch (timed as the
-    // W13 16-row stage), then the tail
+  if (tail && (a->tokens == 1 || (small && !by_env)) && L.hp <= kDecodeHeadMaxK && ceil_div(H / 8, 64) <= 16) {
+    // route + row quantisation + W13 in one launch (timed as the W13 16-row
+    // stage), then the tail
     DecodeHeadArgs h{};
+    h.tokens = (int)a->tokens;
     h.kt = (int)L.kt;
     h.top_k = (int)a->top_k;
     h.shared_id = (int)a->shared_expert_id;
@@ -952,6 +961,52 @@ int bf16_family_forward(const fcmoe_moe_args* a, hipStream_t stream, bool w8) {
   // every token's one route is row t with weight 1, so no route build runs
   // (the route views of fcmoe_bf16_stage_views are then not written).
   const bool dense = smallm_mlp(a, L.routes, w8) && a->top_k == 0 && a->shared_expert_id == 0;
+  // A batch of few routes: two launches. (Whole K chunks, the fused
+  // activations; the one-expert layers have the small-M kernel.)
+  if (!smallm_mlp(a, L.routes, w8) && small_batch(a->tokens, L.routes, H, I, w8 ? 1 : 2) && L.kt <= kDecodeTailSlots &&
+      L.routes <= kWave && H % kmul == 0 && I % kmul == 0 && a->activation != FCMOE_ACT_SWIGLUOAI) {
+    SmallBatchArgs b{};
+    b.tokens = (int)a->tokens;
+    b.kt = (int)L.kt;
+    b.top_k = (int)a->top_k;
+    b.shared_id = (int)a->shared_expert_id;
+    b.ids_is_i64 = a->ids_is_i64;
+    b.valid_experts = (int)a->valid_experts;
+    b.scale_routed = a->shared_expert_id >= 0 && a->top_k > 0 ? 1 : 0;
+    b.scale = a->routed_scaling;
+    b.ids = a->topk_ids;
+    b.topk_w = a->topk_weights;
+    b.x = a->x;
+    b.hidden = H;
+    b.inter = I;
+    b.w13 = a->w13;
+    b.w13_expert_bytes = fcmoe_packed_expert_bytes(w8 ? 1 : 2, 2 * I, H, 2);
+    b.k_chunks13 = (int)(H / kmul);
+    b.n_tiles13 = (int)ceil_div(I, 16);
+    b.w13_scale = a->w13_scale;
+    b.w13_bias = w8 ? nullptr : a->w13_bias;
+    b.activation = a->activation;
+    b.w2 = a->w2;
+    b.w2_expert_bytes = fcmoe_packed_expert_bytes(w8 ? 1 : 2, H, I, 1);
+    b.k_chunks2 = (int)(I / kmul);
+    b.w2_scale = a->w2_scale;
+    b.w2_bias = w8 ? nullptr : a->w2_bias;
+    b.skip_weighted = a->skip_weighted;
+    b.y = L.y;
+    b.route_out = L.route_out;
+    b.route_pos = L.rb.route_pos;
+    b.route_weight = L.rb.route_weight;
+    b.sorted_routes = L.rb.sorted_routes;
+    b.row_token = L.rb.row_token;
+    b.invalid = a->invalid_count ? a->invalid_count : L.rb.invalid;
+    b.out = a->out;
+    {
+      Stage st(FCMOE_STAGE_W13_CLASS0 + class_slot(16), stream);
+      if ((rc = small_batch_bf16_launch(b, w8, false, stream))) return rc;
+    }
+    Stage st(FCMOE_STAGE_W2_CLASS0 + class_slot(16), stream);
+    return small_batch_bf16_launch(b, w8, true, stream);
+  }
   if (!dense) {
     Stage st(FCMOE_STAGE_ROUTE, stream);
     rc = route_launch(a->topk_ids, a->ids_is_i64, a->topk_weights, a->tokens, a->top_k, a->experts,

@@ -16,23 +16,6 @@ namespace fcmoe {
 
 namespace {
 
-template <int Begin, int Count>
-struct TreeSum {
-  __device__ __forceinline__ static float run(const float* v) {
-    constexpr int P = Count > 1 ? [] {
-      int p = 1;
-      while ((p << 1) < Count) p <<= 1;
-      return p;
-    }()
-                                : 1;
-    return TreeSum<Begin, P>::run(v) + TreeSum<Begin + P, Count - P>::run(v);
-  }
-};
-template <int Begin>
-struct TreeSum<Begin, 1> {
-  __device__ __forceinline__ static float run(const float* v) { return v[Begin]; }
-};
-
 // A dropped (invalid) route's row was never written: its leaf is 0 by a
 // select, so whatever the row holds (NaN included) cannot reach the sum.
 template <int K>

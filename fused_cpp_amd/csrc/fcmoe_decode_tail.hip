@@ -39,6 +39,8 @@ constexpr int kQAhead = 2;  // chunks quantised ahead of the MFMA
 constexpr int kQRing = 4;   // per-wave LDS ring of quantised 64-byte chunks
 constexpr int kHeadEarly = 8;  // head: weight chunks issued before the token row is quantised (246 VGPRs: two waves per SIMD)
 
+// ONCE: one token, whose routes' experts differ: nontemporal weight loads.
+template <bool ONCE>
 __global__ __launch_bounds__(kDecodeTailSlots * kWave) void decode_tail_kernel(DecodeTailArgs a) {
   __shared__ float s_val[kDecodeTailSlots][16];
   __shared__ float s_wt[kDecodeTailSlots];
@@ -75,7 +77,8 @@ __global__ __launch_bounds__(kDecodeTailSlots * kWave) void decode_tail_kernel(D
     auto issue = [&](int c, auto slot_c) {
       constexpr int b = decltype(slot_c)::value;
       const int cc = c < kc ? c : kc - 1;
-      bq[b] = __builtin_nontemporal_load((const v4i*)(wb + (int64_t)cc * 1024) + lane);
+      const v4i* src = (const v4i*)(wb + (int64_t)cc * 1024) + lane;
+      bq[b] = ONCE ? __builtin_nontemporal_load(src) : *src;
       yq[b] = yw[(cc * 64 + lane) / 2];
     };
     [&]<int... S>(std::integer_sequence<int, S...>) {
@@ -159,11 +162,11 @@ __global__ __launch_bounds__(kDecodeTailSlots * kWave) void decode_tail_kernel(D
 }
 
 
-// ---- one-token head: route + token-row quantisation + W13 in one launch.
+// ---- head: route + token-row quantisation + W13 in one launch.
 //
-// Workgroup (j, s) is one wave: gate/up channel tile pair j of slot s of the
-// single token. It reads the token's ids, derives its route's sorted position
-// (routes ordered by expert, then by slot: the ascending flat route order of
+// Workgroup (j, r) is one wave: gate/up channel tile pair j of flat route r (at
+// most 64 routes). It reads the batch's ids, derives its route's sorted position
+// (routes ordered by expert, then by flat route: the ascending flat route order of
 // kernels.cpp:583-592) with a ballot, quantises the token row into LDS
 // (quantize_bf16_row, kernels.cpp:211-228) and streams its expert's gate and
 // up tiles through a ring, the row in row 0 of the MFMA as in the tail. The
@@ -172,16 +175,18 @@ __global__ __launch_bounds__(kDecodeTailSlots * kWave) void decode_tail_kernel(D
 // Workgroups j = 0 write the route metadata the tail and the stage views read
 // (route_pos, route_weight, sorted_routes, row_token); (0, 0) writes the
 // invalid-id count.
-template <int CAP>
+template <int CAP, bool ONCE>
 __global__ __launch_bounds__(kWave) void decode_head_kernel(DecodeHeadArgs a) {
   __shared__ __attribute__((aligned(16))) int8_t s_x[kDecodeHeadMaxK];
   const int lane = threadIdx.x;
   const int j = blockIdx.x;
-  const int s = blockIdx.y;
+  const int r = blockIdx.y;  // flat route
+  const int tok = r / a.kt, s = r - tok * a.kt;
+  const int routes = a.tokens * a.kt;  // at most 64: lane l carries route l
 
   // the token row: CAP 16-byte units per lane, in flight with the ids
   const int64_t units = a.hidden / 8;
-  const uint4* xp = (const uint4*)a.x;
+  const uint4* xp = (const uint4*)(a.x + (int64_t)tok * a.hidden);
   uint4 xv[CAP];
 #pragma unroll
   for (int u = 0; u < CAP; ++u) {
@@ -197,34 +202,36 @@ __global__ __launch_bounds__(kWave) void decode_head_kernel(DecodeHeadArgs a) {
   float w_l = 0.0f;
   {
     // unconditional loads, results selected (top_k = 0: no ids, only the shared slot)
-    const int li = lane < a.top_k ? lane : 0;
+    const int lr = lane < routes ? lane : 0;
+    const int lt = lr / a.kt, ls = lr - lt * a.kt;
+    const int li = ls < a.top_k ? lt * a.top_k + ls : 0;
     const int64_t e = a.top_k == 0 ? 0
                       : a.ids_is_i64 ? ((const int64_t*)a.ids)[li]
                                      : (int64_t)((const int32_t*)a.ids)[li];
     float w = a.topk_w && a.top_k > 0 ? a.topk_w[li] : 1.0f;
     if (a.scale_routed) w = w * a.scale;
-    if (lane < a.top_k) {
+    if (lane < routes && ls < a.top_k) {
       ok_l = e >= 0 && e < a.valid_experts;
       e_l = ok_l ? (int)e : 0;
       w_l = w;
-    } else if (lane < a.kt) {
+    } else if (lane < routes) {
       e_l = a.shared_id;
       ok_l = true;
       w_l = 1.0f;
     }
   }
-  const int e_s = __builtin_amdgcn_readlane(e_l, s);
-  const bool ok_s = __builtin_amdgcn_readlane((int)ok_l, s) != 0;
-  const int pos = __popcll(__ballot(ok_l && (e_l < e_s || (e_l == e_s && lane < s))));
-  const int n_invalid = __popcll(__ballot(lane < a.top_k && !ok_l));  // all lanes vote
+  const int e_s = __builtin_amdgcn_readlane(e_l, r);
+  const bool ok_s = __builtin_amdgcn_readlane((int)ok_l, r) != 0;
+  const int pos = __popcll(__ballot(ok_l && (e_l < e_s || (e_l == e_s && lane < r))));
+  const int n_invalid = __popcll(__ballot(lane < routes && !ok_l));  // all lanes vote
   if (j == 0 && lane == 0) {
-    a.route_pos[s] = ok_s ? pos : -1;
-    a.route_weight[s] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_l), s));
+    a.route_pos[r] = ok_s ? pos : -1;
+    a.route_weight[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_l), r));
     if (ok_s) {
-      a.sorted_routes[pos] = s;
-      a.row_token[pos] = 0;
+      a.sorted_routes[pos] = r;
+      a.row_token[pos] = tok;
     }
-    if (s == 0) store_count(a.invalid, n_invalid);
+    if (r == 0) store_count(a.invalid, n_invalid);
   }
   if (!ok_s) return;
 
@@ -237,8 +244,10 @@ __global__ __launch_bounds__(kWave) void decode_head_kernel(DecodeHeadArgs a) {
   auto issue = [&](int c, auto slot_c) {
     constexpr int b = decltype(slot_c)::value;
     const int cc = c < kc ? c : kc - 1;  // past the end: re-read, never consumed
-    bg[b] = __builtin_nontemporal_load((const v4i*)(wg + (int64_t)cc * 1024) + lane);
-    bu[b] = __builtin_nontemporal_load((const v4i*)(wu + (int64_t)cc * 1024) + lane);
+    const v4i* sg = (const v4i*)(wg + (int64_t)cc * 1024) + lane;
+    const v4i* su = (const v4i*)(wu + (int64_t)cc * 1024) + lane;
+    bg[b] = ONCE ? __builtin_nontemporal_load(sg) : *sg;
+    bu[b] = ONCE ? __builtin_nontemporal_load(su) : *su;
   };
   // the first kHeadEarly chunks before the row is quantised, the rest after
   // (all at once, the row's registers and the ring would not fit two waves
@@ -260,7 +269,7 @@ __global__ __launch_bounds__(kWave) void decode_head_kernel(DecodeHeadArgs a) {
   m = wave_max(m);
   const float xs = m > 0.0f ? m / 127.0f : 1.0f;
   const float xinv = 1.0f / xs;
-  if (j == 0 && s == 0 && lane == 0) *a.xs = xs;
+  if (j == 0 && s == 0 && lane == 0) a.xs[tok] = xs;
 #pragma unroll
   for (int u = 0; u < CAP; ++u) {
     const int64_t i = lane + (int64_t)u * kWave;
@@ -335,23 +344,32 @@ int decode_tail_launch(const DecodeTailArgs& a, hipStream_t stream) {
   if (a.kt <= 0 || a.kt > kDecodeTailSlots || a.parts > 2 * kWave || a.k_chunks <= 0 || a.ldq != a.k_chunks * 64 ||
       a.ldy < a.k_chunks * 64 || a.hidden <= 0 || a.tokens > 65535)
     return fail(FCMOE_EINVAL, "decode tail: shapes outside its domain");
-  hipLaunchKernelGGL(decode_tail_kernel, dim3((unsigned)ceil_div(a.hidden, 16), (unsigned)a.tokens),
-                     dim3(a.kt * kWave), 0, stream, a);
+  const dim3 grid((unsigned)ceil_div(a.hidden, 16), (unsigned)a.tokens), block(a.kt * kWave);
+  if (a.tokens == 1)
+    hipLaunchKernelGGL(decode_tail_kernel<true>, grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL(decode_tail_kernel<false>, grid, block, 0, stream, a);
   return check_launch("decode_tail");
 }
 
 int decode_head_launch(const DecodeHeadArgs& a, hipStream_t stream) {
   const int64_t units = ceil_div(a.hidden / 8, kWave);  // x units per lane
-  if (a.kt <= 0 || a.kt > kDecodeTailSlots || a.hidden % 8 || a.k_chunks * 64 > kDecodeHeadMaxK ||
+  if (a.tokens <= 0 || a.kt <= 0 || a.kt > kDecodeTailSlots || (int64_t)a.tokens * a.kt > kWave || a.hidden % 8 || a.k_chunks * 64 > kDecodeHeadMaxK ||
       a.k_chunks * 64 < a.hidden || units > 16 || a.n_tiles <= 0)
     return fail(FCMOE_EINVAL, "decode head: shapes outside its domain");
-  const dim3 grid((unsigned)a.n_tiles, (unsigned)a.kt), block(kWave);
+  const dim3 grid((unsigned)a.n_tiles, (unsigned)(a.tokens * a.kt)), block(kWave);
+  auto launch = [&](auto cap) {
+    if (a.tokens == 1)
+      hipLaunchKernelGGL((decode_head_kernel<decltype(cap)::value, true>), grid, block, 0, stream, a);
+    else
+      hipLaunchKernelGGL((decode_head_kernel<decltype(cap)::value, false>), grid, block, 0, stream, a);
+  };
   if (units <= 4)
-    hipLaunchKernelGGL(decode_head_kernel<4>, grid, block, 0, stream, a);
+    launch(std::integral_constant<int, 4>{});
   else if (units <= 8)
-    hipLaunchKernelGGL(decode_head_kernel<8>, grid, block, 0, stream, a);
+    launch(std::integral_constant<int, 8>{});
   else
-    hipLaunchKernelGGL(decode_head_kernel<16>, grid, block, 0, stream, a);
+    launch(std::integral_constant<int, 16>{});
   return check_launch("decode_head");
 }
 

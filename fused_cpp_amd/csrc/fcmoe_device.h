@@ -128,6 +128,25 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// The BF16 merge's sum of Count values: adjacent ranges split at the largest
+// power of two below the length (route_merge.cpp:47-86).
+template <int Begin, int Count>
+struct TreeSum {
+  __device__ __forceinline__ static float run(const float* v) {
+    constexpr int P = Count > 1 ? [] {
+      int p = 1;
+      while ((p << 1) < Count) p <<= 1;
+      return p;
+    }()
+                                : 1;
+    return TreeSum<Begin, P>::run(v) + TreeSum<Begin + P, Count - P>::run(v);
+  }
+};
+template <int Begin>
+struct TreeSum<Begin, 1> {
+  __device__ __forceinline__ static float run(const float* v) { return v[Begin]; }
+};
+
 __host__ __device__ __forceinline__ int64_t round_up(int64_t v, int64_t q) { return (v + q - 1) / q * q; }
 __host__ __device__ __forceinline__ int64_t ceil_div(int64_t v, int64_t q) { return (v + q - 1) / q; }
 

@@ -309,16 +309,17 @@ struct DecodeTailArgs {
   uint16_t* out;               // [tokens, hidden] bf16
 };
 int decode_tail_launch(const DecodeTailArgs& a, hipStream_t stream);
-// One-token head: route + token-row quantisation + W13 in one launch; writes
+// Head: route + token-row quantisation + W13 in one launch (at most 64 routes); writes
 // y, rowpart and the route metadata (route_pos, route_weight, sorted_routes,
 // row_token, the invalid count) as the route and W13 launches do.
 constexpr int64_t kDecodeHeadMaxK = 8192;  // padded hidden size it takes (the row lives in LDS)
 struct DecodeHeadArgs {
+  int tokens;                // tokens * kt at most 64
   int kt, top_k, shared_id, ids_is_i64, valid_experts, scale_routed;
   float scale;
-  const void* ids;           // [top_k] the token's ids
-  const float* topk_w;       // [top_k] or null (weights 1)
-  const uint16_t* x;         // [hidden] bf16 token row
+  const void* ids;           // [tokens, top_k]
+  const float* topk_w;       // [tokens, top_k] or null (weights 1)
+  const uint16_t* x;         // [tokens, hidden] bf16 token rows
   int64_t hidden;
   const void* w;             // packed W13 [E][2 groups][n_tiles][k_chunks][1 KB]
   int64_t w_expert_bytes;
@@ -329,13 +330,47 @@ struct DecodeHeadArgs {
   uint16_t* y;               // [positions, ldy]
   int64_t ldy;
   float* rowpart;            // [positions, n_tiles]
-  float* xs;                 // [1] the token row's scale
-  int32_t* route_pos;        // [kt]
-  float* route_weight;       // [kt]
-  int32_t* sorted_routes;    // [kt]
-  int32_t* row_token;        // [kt]
+  float* xs;                 // [tokens] the token rows' scales
+  int32_t* route_pos;        // [tokens * kt]
+  float* route_weight;       // [tokens * kt]
+  int32_t* sorted_routes;    // [tokens * kt]
+  int32_t* row_token;        // [tokens * kt]
   int32_t* invalid;          // [1]
 };
 int decode_head_launch(const DecodeHeadArgs& a, hipStream_t stream);
+
+// ---- BF16 / W8A16 layers of at most 64 routes (fcmoe_decode_bf16.hip) ----
+// Route build + W13 + activation, then W2 + merge: two launches. H and F are
+// multiples of a K chunk (32 elements, W8A16 64). Writes out, y, the route_out
+// view and the route metadata as the launches it stands for.
+struct SmallBatchArgs {
+  int tokens, kt, top_k, shared_id, ids_is_i64, valid_experts, scale_routed;
+  float scale;
+  const void* ids;             // [tokens, top_k]
+  const float* topk_w;         // [tokens, top_k]
+  const uint16_t* x;           // [tokens, hidden] bf16
+  int64_t hidden, inter;
+  const void* w13;             // packed [E][2 groups][n_tiles13][k_chunks13][1 KB]
+  int64_t w13_expert_bytes;
+  int k_chunks13, n_tiles13;
+  const float* w13_scale;      // W8A16 [E, 2 inter]
+  const float* w13_bias;       // BF16, optional [E, 2 inter]
+  int activation;
+  const void* w2;              // packed [E][ceil(hidden / 16)][k_chunks2][1 KB]
+  int64_t w2_expert_bytes;
+  int k_chunks2;
+  const float* w2_scale;       // W8A16 [E, hidden]
+  const float* w2_bias;        // BF16, optional [E, hidden]
+  int skip_weighted;
+  uint16_t* y;                 // [routes, inter] by sorted position
+  float* route_out;            // [routes, hidden] by flat route
+  int32_t* route_pos;
+  float* route_weight;
+  int32_t* sorted_routes;
+  int32_t* row_token;
+  int32_t* invalid;
+  uint16_t* out;               // [tokens, hidden] bf16
+};
+int small_batch_bf16_launch(const SmallBatchArgs& a, bool w8, bool tail, hipStream_t stream);
 
 }  // namespace fcmoe
