@@ -185,11 +185,16 @@ typedef __attribute__((address_space(3))) uint8_t* lds_u8_ptr;
 
 template <int FN>
 constexpr int staged_slice_bytes(int epi) {
-  return epi == kEpiW13SwigluI8 ? 16 * ((FN / 2) * 32 + 16) + 16 * (FN / 2) * 4 : 16 * (FN * 64 + 16);
+  return epi_pair(epi) ? 16 * ((FN / 2) * 32 + 16) + (epi == kEpiW13SwigluI8 ? 16 * (FN / 2) * 4 : 0)
+                       : 16 * (FN * 64 + 16);
+}
+constexpr bool epi_staged(int epi) {
+  return epi == kEpiW13SwigluI8 || epi == kEpiW2RouteI8 || epi == kEpiI8Gemm || epi == kEpiW13ActBf16 ||
+         epi == kEpiW2RouteBf16 || epi == kEpiW13ActW8 || epi == kEpiW2RouteW8;
 }
 
-template <int EPI, int FM, int FN>
-__device__ __forceinline__ void staged_epilogue(const GemmParams& p, const v4i (&acc)[FM][FN],
+template <int EPI, int FM, int FN, typename AccT>
+__device__ __forceinline__ void staged_epilogue(const GemmParams& p, const AccT (&acc)[FM][FN],
                                                 const int64_t (&gtile)[FN], const bool (&tvalid)[FN], int row_base,
                                                 int rows, int pos0, int expert, int lane, const EpiMeta& m,
                                                 lds_u8_ptr slice) {
@@ -286,6 +291,108 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams& p, const v4i (
         if (r < rows && t < p.n_tiles)
           p.rowpart[(int64_t)(pos0 + r) * p.n_tiles + t] =
               *(__attribute__((address_space(3))) const float*)(rp + lane * 4);
+      }
+    }
+  } else if constexpr (EPI == kEpiW13ActBf16 || EPI == kEpiW13ActW8) {
+    // The BF16 and W8A16 activations (the generic epilogue's arithmetic),
+    // stored as row-contiguous 16-byte pieces of 8 channels. Channels past F
+    // are left alone: y is zero there for the padded K of W2.
+    constexpr int HP = FN / 2;
+    constexpr int RS = HP * 32 + 16;
+    constexpr int UPR = HP * 2;
+    float cg[HP], cu[HP];
+    const float* cv = EPI == kEpiW13ActW8 ? p.scale_col : p.bias;
+#pragma unroll
+    for (int j = 0; j < HP; ++j) {
+      const int64_t f = gtile[j] * 16 + col;
+      const int64_t fc = tvalid[j] && f < p.n_half ? f : 0;
+      cg[j] = cv ? cv[(int64_t)expert * p.n + fc] : 0.0f;
+      cu[j] = cv ? cv[(int64_t)expert * p.n + p.n_half + fc] : 0.0f;
+    }
+    const int64_t f0 = gtile[0] * 16;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int rbase = row_base + i * 16;
+      if (rbase >= rows) break;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < HP; ++j) {
+          float gate = acc[i][j][q], up = acc[i][j + HP][q];
+          if constexpr (EPI == kEpiW13ActW8) {
+            gate = gate * cg[j];
+            up = up * cu[j];
+          } else if (p.bias) {
+            gate = gate + cg[j];
+            up = up + cu[j];
+          }
+          *(__attribute__((address_space(3))) uint16_t*)(slice + (rq + q) * RS + (j * 16 + col) * 2) =
+              f32_to_bf16(act_bf16_mode(gate, up, p.activation));
+        }
+#pragma unroll
+      for (int h = 0; h < (16 * UPR + kWave - 1) / kWave; ++h) {
+        const int idx = h * kWave + lane;
+        const int row = idx / UPR, u = idx % UPR;
+        const int r = rbase + row;
+        const int64_t ch = f0 + u * 8;
+        if (idx < 16 * UPR && r < rows && ch < p.n_half) {
+          uint16_t* dst = (uint16_t*)p.out + (int64_t)(pos0 + r) * p.ldo + ch;
+          const lds_u8_ptr src = slice + row * RS + u * 16;
+          if (ch + 8 <= p.n_half) {
+            *(v4i*)dst = *(__attribute__((address_space(3))) const v4i*)src;
+          } else {
+            for (int e = 0; ch + e < p.n_half; ++e) dst[e] = ((__attribute__((address_space(3))) const uint16_t*)src)[e];
+          }
+        }
+      }
+    }
+  } else if constexpr (EPI == kEpiW2RouteBf16 || EPI == kEpiW2RouteW8) {
+    // The W2 route rows of BF16 and W8A16, as the int8 ones below: fp32 staged,
+    // stored nontemporal in 16-byte pieces (channel by channel where H is not a
+    // multiple of 4). With the W13 rows above, against one store per lane and
+    // accumulator: BF16 TP rank (H 4096, F 512) T=2047 307 -> 293 us, T=4000 569
+    // -> 523, W8A16 T=4000 522 -> 484; DSv3 W8A16 T=2048 2622 -> 2568.
+    constexpr int RS = FN * 64 + 16;
+    constexpr int UPR = FN * 4;
+    float cs[FN];
+    const float* cv = EPI == kEpiW2RouteW8 ? p.scale_col : p.bias;
+    const int64_t c0 = gtile[0] * 16;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int64_t ch = c0 + j * 16 + col;
+      cs[j] = cv ? cv[(int64_t)expert * p.n + (tvalid[j] && ch < p.n ? ch : 0)] : 0.0f;
+    }
+    const bool vec = p.ldo % 4 == 0;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int rbase = row_base + i * 16;
+      if (rbase >= rows) break;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          float v = acc[i][j][q];
+          if constexpr (EPI == kEpiW2RouteW8)
+            v = v * cs[j];
+          else if (p.bias)
+            v = v + cs[j];
+          *(__attribute__((address_space(3))) float*)(slice + (rq + q) * RS + (j * 16 + col) * 4) = v;
+        }
+#pragma unroll
+      for (int h = 0; h < 16 * UPR / kWave; ++h) {
+        const int idx = h * kWave + lane;
+        const int row = idx / UPR, u = idx % UPR;
+        const int r = rbase + row;
+        const int64_t ch = c0 + u * 4;
+        if (r < rows && ch < p.n) {
+          float* dst = (float*)p.out + (int64_t)m.orow[r] * p.ldo + ch;
+          const v4i v = *(__attribute__((address_space(3))) const v4i*)(slice + row * RS + u * 16);
+          if (vec) {
+            __builtin_nontemporal_store(v, (v4i*)dst);
+          } else {
+            for (int e = 0; e < 4 && ch + e < p.n; ++e) dst[e] = __int_as_float(v[e]);
+          }
+        }
       }
     }
   } else if constexpr (EPI == kEpiI8Gemm) {
@@ -868,7 +975,7 @@ __device__ __forceinline__ void lds_gemm_body(const GemmParams& p, int n_blocks,
 #pragma unroll
   for (int j = 0; j < FN; ++j) gtile[j] = tile_of(wn, j, &tvalid[j]);
   const EpiMeta meta{(lds_cfloat_ptr)meta_rs, (lds_cint_ptr)meta_orow, (lds_cfloat_ptr)meta_cs, wn * FN};
-  if constexpr (EPI == kEpiW13SwigluI8 || EPI == kEpiW2RouteI8 || EPI == kEpiI8Gemm) {
+  if constexpr (epi_staged(EPI)) {
     static_assert(WAVES * staged_slice_bytes<FN>(EPI) <= SA * A_BYTES + SB * B_BYTES, "staging slices fit the stages");
     // every wave is past its last chunk's fragment reads: the stages are free
     __builtin_amdgcn_s_barrier();
