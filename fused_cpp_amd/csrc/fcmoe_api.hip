@@ -55,10 +55,11 @@ int class_slot(int bm) {
 //   * 64-row tiles (fcmoe_gemm_mid.hip) from there to r = 48, and beyond it
 //     while the layer's operations are few: what a larger tile would save in
 //     weight re-reads is less than what its longer K walk on a few dozen
-//     workgroups costs. TP W8A8 T=200 180 -> 66, T=1000 244 -> 146; BF16 T=200
-//     253 -> 94, T=1000 322 -> 225; W8A16 T=400 246 -> 88 (the start's side:
-//     class launches on forked streams). The operations bound: TP BF16 T=1000
-//     (88 GFLOP) 225 against 257 on 128 rows, T=2047 (180) 422 against 319;
+//     workgroups costs. TP W8A8 T=200 180 -> 55, T=1000 244 -> 146; BF16 T=200
+//     253 -> 94, T=1000 322 -> 225; W8A16 T=400 246 -> 88 (the larger figure:
+//     128-row and larger class launches on forked streams). The operations bound: TP BF16 T=1000
+//     (88 GFLOP) 225 against 257 on 128 rows, T=2047 (180) 422 against 319 (293
+//     with the staged epilogue);
 //     one BF16 expert at 1000 rows (88) 246 against 288, at 2000 (180) 478
 //     against 332; 8 DSv3 W8A8 experts at T=256 (203 GOP) 298 against 181.
 //   * 128-row tiles above; 256-row ones when experts hold many tiles of either

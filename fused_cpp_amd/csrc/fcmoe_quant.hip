@@ -2,9 +2,9 @@
 // BF16 activation pass.
 //
 // Row kernels: bf16 activation rows (cols % 8 == 0, up to 16384 columns) use
-// one workgroup per row with the row held in registers; other rows use one
-// wavefront per row (a strided max|x| pass, a butterfly, then the quantise
-// pass). These are HBM-bound byte kernels (2 bytes in, 1 byte out per element).
+// one workgroup per row with the row held in registers, and so do fp32 rows and
+// bf16 rows of any width; many narrow rows and wider ones use one wavefront per
+// row (a strided max|x| pass, a butterfly, then the quantise pass). These are HBM-bound byte kernels (2 bytes in, 1 byte out per element).
 #include <type_traits>
 
 #include "fcmoe_device.h"
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kRowsPerBlock * kWave) void quant_rows_kernel(const
 }
 
 // bf16 rows with cols % 8 == 0 and ldq % 8 == 0 (every activation row of the
-// MoE and i8gemm paths): one kRowThreads workgroup per row (quant_row_wg).
+// MoE paths): one kRowThreads workgroup per row (quant_row_wg).
 template <int CAP>
 __global__ __launch_bounds__(kRowThreads) void quant_rows_wg_kernel(const uint16_t* x, int64_t cols, int rounding,
                                                                      int8_t* q, int64_t ldq, float* scales) {

@@ -1,6 +1,6 @@
 // fcmoe_quant_row.h -- per-row activation quantisation shared by the row
-// quantisation kernel (fcmoe_quant.hip) and the small-batch route kernel that
-// also quantises the token rows (fcmoe_route.hip).
+// quantisation kernels (fcmoe_quant.hip), the route launches that also quantise
+// the token rows (fcmoe_route.hip) and the decode head (fcmoe_decode_tail.hip).
 #pragma once
 
 #include "fcmoe_device.h"
