@@ -85,9 +85,11 @@ template <bool W8, bool ONCE>
 __global__ __launch_bounds__(kWave) void bf16_head_kernel(SmallBatchArgs a) {
   const int lane = threadIdx.x;
   const int j = blockIdx.x, r = blockIdx.y;
-  const int routes = a.tokens * a.kt;  // at most 64: lane l carries route l
+  const int tok = ONCE ? 0 : r / a.kt;  // (ONCE is one token: no division ahead of the loads)
+  const int routes = ONCE ? a.kt : a.tokens * a.kt;  // at most 64: lane l carries route l
   // every route's expert, validity (route_expert) and combined weight (route_weight_of)
-  const int lt = (lane < routes ? lane : 0) / a.kt, ls = (lane < routes ? lane : 0) % a.kt;
+  const int lr = lane < routes ? lane : 0;
+  const int lt = ONCE ? 0 : lr / a.kt, ls = lr - lt * a.kt;
   const int idx = ls < a.top_k ? lt * a.top_k + ls : 0;  // (top_k = 0: no ids, only the shared slot)
   const int64_t e = a.top_k == 0 ? 0 : a.ids_is_i64 ? ((const int64_t*)a.ids)[idx] : (int64_t)((const int32_t*)a.ids)[idx];
   float w_l = a.topk_w && a.top_k > 0 ? a.topk_w[idx] : 1.0f;
@@ -109,7 +111,7 @@ __global__ __launch_bounds__(kWave) void bf16_head_kernel(SmallBatchArgs a) {
     a.route_weight[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_l), r));
     if (ok_r) {
       a.sorted_routes[pos] = r;
-      a.row_token[pos] = r / a.kt;
+      a.row_token[pos] = tok;
     }
     if (r == 0) store_count(a.invalid, n_invalid);
   }
@@ -127,7 +129,7 @@ __global__ __launch_bounds__(kWave) void bf16_head_kernel(SmallBatchArgs a) {
     cu = cv[(int64_t)e_r * 2 * a.inter + a.inter + fc];
   }
   v4f acc[2];
-  row_times_tiles<W8, ONCE, 2>((const uint8_t*)(a.x + (int64_t)(r / a.kt) * a.hidden), w, kc, lane, acc);
+  row_times_tiles<W8, ONCE, 2>((const uint8_t*)(a.x + (int64_t)tok * a.hidden), w, kc, lane, acc);
   if (lane >= 16 || f >= a.inter) return;
   float gate = acc[0][0], up = acc[1][0];
   if constexpr (W8) {

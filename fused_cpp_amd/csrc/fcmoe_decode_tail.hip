@@ -181,8 +181,10 @@ __global__ __launch_bounds__(kWave) void decode_head_kernel(DecodeHeadArgs a) {
   const int lane = threadIdx.x;
   const int j = blockIdx.x;
   const int r = blockIdx.y;  // flat route
-  const int tok = r / a.kt, s = r - tok * a.kt;
-  const int routes = a.tokens * a.kt;  // at most 64: lane l carries route l
+  // ONCE is one token: the divisions by kt, ahead of the ids' and weights' loads
+  // in every workgroup, cost a one-token DSv3 layer 0.4 of 70 us
+  const int tok = ONCE ? 0 : r / a.kt, s = r - tok * a.kt;
+  const int routes = ONCE ? a.kt : a.tokens * a.kt;  // at most 64: lane l carries route l
 
   // the token row: CAP 16-byte units per lane, in flight with the ids
   const int64_t units = a.hidden / 8;
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(kWave) void decode_head_kernel(DecodeHeadArgs a) {
   {
     // unconditional loads, results selected (top_k = 0: no ids, only the shared slot)
     const int lr = lane < routes ? lane : 0;
-    const int lt = lr / a.kt, ls = lr - lt * a.kt;
+    const int lt = ONCE ? 0 : lr / a.kt, ls = lr - lt * a.kt;
     const int li = ls < a.top_k ? lt * a.top_k + ls : 0;
     const int64_t e = a.top_k == 0 ? 0
                       : a.ids_is_i64 ? ((const int64_t*)a.ids)[li]
