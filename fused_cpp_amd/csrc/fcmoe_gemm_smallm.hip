@@ -180,9 +180,13 @@ __device__ __forceinline__ void smallm_body(const SmallMArgs& p, int bx, int by)
   [&]<int... S>(std::integer_sequence<int, S...>) {
     (issue(S, std::integral_constant<int, S>{}), ...);
   }(std::make_integer_sequence<int, D - 1>{});
-  // the K loop's first barrier publishes the rows' scales
-  if constexpr (I8)
+  // The K loop's first barrier publishes the rows' scales: their write ends
+  // here (lgkmcnt(0); the ring's loads stay in flight), as that barrier waits
+  // for none and with one chunk it is the only one before the epilogue.
+  if constexpr (I8) {
     if (threadIdx.x < FM * 16) srow[threadIdx.x] = rscale;
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+  }
 
   // Chunk t's fragments and MFMAs. The scheduling barrier keeps the MFMAs, and
   // with them the waits for this wave's fragment reads, ahead of the next

@@ -126,31 +126,40 @@ def smallm_asm(tmp_path_factory) -> str:
     return out.read_text()
 
 
-def test_small_m_stage_reads_end_before_the_barrier(smallm_asm):
+def _lds_accesses_end_before_the_barrier(name: str, body: list[str]) -> int:
+    """No LDS read or write is pending at a barrier; returns the number of barriers."""
+    pending = []
+    barriers = 0
+    for line in body:
+        op = line.strip()
+        if op.startswith("ds_"):
+            pending.append(op.split()[0])
+        elif op.startswith("s_waitcnt") and "lgkmcnt(0)" in op:
+            pending = []
+        elif op.startswith("s_barrier"):
+            barriers += 1
+            assert not pending, (name, barriers, pending)
+    return barriers
+
+
+def _barriers_after_the_last_load(body: list[str]) -> int:
+    last_load = max(i for i, line in enumerate(body) if "buffer_load" in line)
+    return sum(line.strip().startswith("s_barrier") for line in body[last_load:])
+
+
+def test_small_m_lds_accesses_end_before_the_barrier(smallm_asm):
     """The small-M kernel's stages are refilled right after the workgroup
-    barrier, so no fragment read may still be queued when a wave reaches it:
-    a wait for every LDS read lies between the last read and the barrier. And
-    the steps after the K loop issue no loads, so that their vmcnt counts are
-    the ones the source computes."""
+    barrier, so no fragment read may still be queued when a wave reaches it, and
+    the row scales are published by the K loop's first barrier (with one chunk
+    the only one), so their write may not be either: a wait for every LDS access
+    lies between it and the barrier. And the steps after the K loop issue no
+    loads, so that their vmcnt counts are the ones the source computes."""
     kernels = re.findall(r"^(_Z\w*smallm_(?:pair_)?kernel\w*):(.*?)\.Lfunc_end", smallm_asm, re.M | re.S)
     assert len(kernels) >= 15
     for name, text in kernels:
         body = text.splitlines()
-        pending = False
-        barriers = 0
-        for line in body:
-            op = line.strip()
-            if op.startswith("ds_read"):
-                pending = True
-            elif op.startswith("s_waitcnt") and "lgkmcnt(0)" in op:
-                pending = False
-            elif op.startswith("s_barrier"):
-                barriers += 1
-                assert not pending, (name, barriers)
-        assert barriers >= 15, name
-        last_loop_load = max(i for i, line in enumerate(body) if "buffer_load" in line)
-        later = [i for i, line in enumerate(body) if line.strip().startswith("s_barrier") and i > last_loop_load]
-        assert len(later) >= 7, (name, len(later))
+        assert _lds_accesses_end_before_the_barrier(name, body) >= 15, name
+        assert _barriers_after_the_last_load(body) >= 7, name
 
 
 def test_mixed_plan_register_budget(lds_asm, tmp_path):
