@@ -184,12 +184,15 @@ __global__ __launch_bounds__(kMidWaves * kWave) void grouped_gemm_mid_kernel(Gem
     (issue(S, std::integral_constant<int, S>{}), ...);
   }(std::make_integer_sequence<int, D - 1>{});
 
-  // Published by the K loop's first barrier. Every thread writes its entry (the
+  // Published by the K loop's first barrier, with one chunk the only one: the
+  // writes end here (lgkmcnt(0); the ring's loads stay in flight), as the
+  // loop's barriers wait for none. Every thread writes its entry (the
   // epilogue reads the first BM and 16 NT): in a conditional block the loads
   // would be sunk into it, behind the ring, and drain it.
   meta_rs[mt] = m_rs;
   meta_orow[mt] = m_orow;
   meta_cs[mt] = m_cs;
+  __builtin_amdgcn_s_waitcnt(0xC07F);
 
   // The closing scheduling barrier keeps the MFMAs, and with them the waits
   // for this wave's fragment reads, ahead of the next chunk's workgroup

@@ -114,16 +114,25 @@ def _vgprs(asm: str) -> dict[str, int]:
     return dict(zip(names, counts))
 
 
-@pytest.fixture(scope="module")
-def smallm_asm(tmp_path_factory) -> str:
+def _device_asm(tmp_path_factory, stem: str) -> str:
     hipcc = ROCM / "bin" / "hipcc"
     if not hipcc.exists():
         pytest.skip("hipcc not available")
-    out = tmp_path_factory.mktemp("isa") / "fcmoe_gemm_smallm.s"
-    proc = subprocess.run([str(hipcc), *HIP_FLAGS, "--cuda-device-only", "-S", str(CSRC / "fcmoe_gemm_smallm.hip"),
+    out = tmp_path_factory.mktemp("isa") / f"{stem}.s"
+    proc = subprocess.run([str(hipcc), *HIP_FLAGS, "--cuda-device-only", "-S", str(CSRC / f"{stem}.hip"),
                            "-o", str(out)], capture_output=True, text=True)
     assert proc.returncode == 0, proc.stdout + proc.stderr
     return out.read_text()
+
+
+@pytest.fixture(scope="module")
+def smallm_asm(tmp_path_factory) -> str:
+    return _device_asm(tmp_path_factory, "fcmoe_gemm_smallm")
+
+
+@pytest.fixture(scope="module")
+def mid_asm(tmp_path_factory) -> str:
+    return _device_asm(tmp_path_factory, "fcmoe_gemm_mid")
 
 
 def _lds_accesses_end_before_the_barrier(name: str, body: list[str]) -> int:
@@ -160,6 +169,19 @@ def test_small_m_lds_accesses_end_before_the_barrier(smallm_asm):
         body = text.splitlines()
         assert _lds_accesses_end_before_the_barrier(name, body) >= 15, name
         assert _barriers_after_the_last_load(body) >= 7, name
+
+
+def test_mid_lds_accesses_end_before_the_barrier(mid_asm):
+    """The same two invariants of the 64-row tiles: their stages are refilled
+    after the barrier too, and the first barrier publishes the epilogue's row
+    scales, output rows and channel scales. (Rings of 8 chunks; W8A16 of 6.)"""
+    kernels = re.findall(r"^(_Z\w*grouped_gemm_mid_kernel\w*):(.*?)\.Lfunc_end", mid_asm, re.M | re.S)
+    assert len(kernels) >= 14
+    for name, text in kernels:
+        body = text.splitlines()
+        depth = 6 if re.search(r"ILb0ELi[78]E", name) else 8
+        assert _lds_accesses_end_before_the_barrier(name, body) >= 2 * depth - 1, name
+        assert _barriers_after_the_last_load(body) >= depth - 1, name
 
 
 def test_mixed_plan_register_budget(lds_asm, tmp_path):
