@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <initializer_list>
+#include <iterator>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -97,20 +98,35 @@ int64_t small_rows() {
 
 bool weights_once(const MoeShape& m) { return m.few_rows(48) && m.weight_bytes() > kCachedWeights; }
 
-// FCMOE_TILE_CLASSES (tile rows in rising order, "128,192,256"): this class set
-// instead of the chosen one, so that tests and measurements reach every tile
-// at any shape; an unknown size is refused by its launch. Read on every call.
+// FCMOE_TILE_CLASSES (tile rows in strictly rising order, "128,192,256"): this
+// class set instead of the chosen one, so that tests and measurements reach
+// every tile at any shape. Read on every call. Returns the number of classes,
+// 0 when it is not set and -1 when it is not such a list of kClassBM sizes
+// (check_shapes then refuses the call).
+int forced_classes(int (&bms)[kMaxClasses]) {
+  const char* v = getenv("FCMOE_TILE_CLASSES");
+  if (!v || !v[0]) return 0;
+  for (int n = 0; n < kMaxClasses; ++v) {
+    char* end;
+    const long bm = strtol(v, &end, 10);
+    const bool known = std::find(std::begin(kClassBM), std::end(kClassBM), bm) != std::end(kClassBM);
+    if (end == v || !known || (n > 0 && bm <= bms[n - 1])) return -1;
+    bms[n++] = (int)bm;
+    if (!*end) return n;
+    if (*end != ',') return -1;
+    v = end;
+  }
+  return -1;
+}
+
 // lds: the tiles above 32 rows can address A and one expert's weights (W8A16
 // has no other kernel for them).
 TileClasses select_classes(const MoeShape& m, bool lds = true) {
   auto set = [&](std::initializer_list<int> bms) {
     return make_tile_classes(bms.begin(), (int)bms.size(), m.routes, m.experts);
   };
-  if (const char* v = getenv("FCMOE_TILE_CLASSES"); v && v[0] && lds) {
-    int bms[kMaxClasses], n = 0;
-    for (char* end; n < kMaxClasses && *v; v = *end ? end + 1 : end) bms[n++] = (int)strtol(v, &end, 10);
-    return make_tile_classes(bms, n, m.routes, m.experts);
-  }
+  if (int bms[kMaxClasses]; lds)
+    if (const int n = forced_classes(bms); n > 0) return make_tile_classes(bms, n, m.routes, m.experts);
   const bool tiny = m.routes <= small_rows();
   if (m.family == kW8A16 && !lds) return tiny || m.few_rows(8) ? set({16}) : set({16, 32});
   const bool big = m.weight_bytes() > kBigWeights;
@@ -171,6 +187,8 @@ int check_shapes(const fcmoe_moe_args* a) {
   if (a->valid_experts <= 0 || a->valid_experts > a->experts) return fail(FCMOE_EINVAL, "bad valid_experts");
   if (a->shared_expert_id >= a->experts) return fail(FCMOE_EINVAL, "shared_expert_id out of range");
   if (a->tokens > (int64_t)1 << 24) return fail(FCMOE_EINVAL, "tokens must be <= 2^24");
+  if (int bms[kMaxClasses]; forced_classes(bms) < 0)
+    return fail(FCMOE_EINVAL, "FCMOE_TILE_CLASSES must list sizes of 16,32,64,128,192,256 in rising order");
   return FCMOE_OK;
 }
 
@@ -585,7 +603,8 @@ bool small_batch(int64_t tokens, int64_t routes, int64_t hidden, int64_t inter, 
 // classic launches only.
 int run_w8a8_stage(const TileClasses& tc, const RouteBuffers& rb, int epi, const GemmParams& base, int stage0,
                    int stage_mixed, bool serial, hipStream_t stream) {
-  const bool prefill = tc.n == 4 && tc.bm[0] == 16 && tc.bm[3] == 256;
+  const bool prefill =
+      tc.n == kNumPrefillClasses && std::equal(std::begin(kPrefillClassBM), std::end(kPrefillClassBM), tc.bm);
   GemmParams gate = base;
   if (prefill) {
     gate.plan_tiles = rb.tile_count;  // class 0: the 16-row tiles

@@ -7,6 +7,8 @@ from __future__ import annotations
 
 import ctypes
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -59,6 +61,38 @@ def test_cabi_library_exports_every_declared_symbol():
     missing = [name for name in sorted(declared) if not hasattr(lib, name)]
     assert not missing, f"libfcmoe.so lacks {missing}"
     assert set(cabi.SIGNATURES) == declared  # the ctypes binding covers the whole header
+
+
+@pytest.mark.parametrize("classes", ["0", "abc", "128,", "128, ", ",", "64,0", "-16", "48", "128,64", "64,64", "64;128",
+                                     "16,32,64,128,192,256,256"])
+def test_malformed_tile_classes_are_refused(monkeypatch, classes):
+    """FCMOE_TILE_CLASSES must list known tile sizes in strictly rising order: a size of 0 would divide
+    by zero on the host, already in the workspace query, so the check runs in a process of its own."""
+    code = """
+import ctypes
+from fused_cpp_amd import cabi
+L = cabi.lib()
+a = cabi.MoeArgs()
+a.tokens, a.hidden, a.inter, a.top_k, a.experts, a.valid_experts, a.shared_expert_id = 64, 256, 128, 2, 8, 8, -1
+a.activation = cabi.FCMOE_ACT_SILU_CLAMP10
+for family in ("w8a8", "bf16", "w8a16"):
+    assert getattr(L, f"fcmoe_{family}_workspace_bytes")(ctypes.byref(a)) == 0, family
+    assert getattr(L, f"fcmoe_{family}_forward")(ctypes.byref(a), None) == -1, family
+    assert b"FCMOE_TILE_CLASSES" in L.fcmoe_last_error()
+"""
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
+    proc = subprocess.run([sys.executable, "-c", code], cwd=REPO, capture_output=True, text=True)
+    assert proc.returncode == 0, (proc.returncode, proc.stderr)
+
+
+@pytest.mark.parametrize("classes", ["16", "64", "128,192,256", "16,32,64,128,192,256"])
+def test_tile_classes_of_known_sizes_are_accepted(monkeypatch, classes):
+    from fused_cpp_amd import cabi
+
+    a = cabi.MoeArgs()
+    a.tokens, a.hidden, a.inter, a.top_k, a.experts, a.valid_experts, a.shared_expert_id = 64, 256, 128, 2, 8, 8, -1
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
+    assert cabi.lib().fcmoe_w8a8_workspace_bytes(ctypes.byref(a)) > 0
 
 
 def test_cabi_host_only_calls():
