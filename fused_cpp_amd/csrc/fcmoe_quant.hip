@@ -320,8 +320,9 @@ int quant_rows_launch(const void* x, int x_is_f32, int64_t rows, int64_t cols, i
   }
   // Many narrow rows leave most of a workgroup idle and stay on one wave per
   // row: 16384 rows of 250 9.9 us there against 11.1, of 500 16.6 against 14.0;
-  // 2048 rows of 33 2.55 against 2.88, 300 rows 2.41 against 2.24.
-  if (rows <= INT32_MAX && (rows <= 1024 || cols > 320)) {
+  // 2048 rows of 33 2.55 against 2.88, 300 rows 2.41 against 2.24. So do more
+  // rows than one launch has workgroups of kRowThreads (under 2^32 threads).
+  if (rows <= (int64_t)(UINT32_MAX / kRowThreads) && (rows <= 1024 || cols > 320)) {
     const dim3 grid((unsigned)rows), block(kRowThreads);
     bool done;
     if (x_is_f32 && cols % 4 == 0 && ldq % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)q % 4 == 0)

@@ -57,3 +57,25 @@ def test_quant_rows_of_fp32_off_16_bytes(gpu, oracle_lib):
     rq, rs = oracle_lib.quant_rows_even(x)
     np.testing.assert_array_equal(q[1:].cpu().numpy().reshape(4, 64), rq)
     np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), rs.view(np.uint32))
+
+
+def test_quant_rows_past_one_launch_of_row_workgroups(gpu, oracle_lib):
+    """2^24 rows: a workgroup of 256 threads per row would be 2^32 threads, more than a launch may have."""
+    import torch
+
+    from fused_cpp_amd import cabi
+
+    rows, cols = 1 << 24, 321
+    x = torch.zeros((rows, cols), dtype=torch.bfloat16, device=gpu)
+    at = [0, 1, 4095, rows // 2, rows - 2, rows - 1]
+    xr = H.bits_to_f32(H.bf16_bits(np.random.default_rng(3).standard_normal((len(at), cols)).astype(np.float32)))
+    x[at] = torch.from_numpy(xr).to(gpu).to(torch.bfloat16)
+    q = torch.full((rows, cols), 99, dtype=torch.int8, device=gpu)
+    s = torch.zeros(rows, device=gpu)
+    cabi.check(cabi.lib().fcmoe_quantize_rows(x.data_ptr(), 0, rows, cols, 1, q.data_ptr(), cols, s.data_ptr(),
+                                              cabi.stream_handle()), "quantize_rows")
+    rq, rs = oracle_lib.quant_rows_even(H.bf16_bits(xr))
+    np.testing.assert_array_equal(q[at].cpu().numpy(), rq)
+    np.testing.assert_array_equal(s[at].cpu().numpy().view(np.uint32), rs.view(np.uint32))
+    assert int((s == 1).sum()) == rows - len(at)  # rows of zeros: scale 1, bytes 0
+    assert not q[2:4095].any()
