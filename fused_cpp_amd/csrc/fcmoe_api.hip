@@ -1034,13 +1034,18 @@ int bf16_family_forward(const fcmoe_moe_args* a, hipStream_t stream, bool w8) {
                       a->shared_expert_id >= 0 && a->top_k > 0, L.rb, L.tc, a->invalid_count, stream);
     if (rc) return rc;
   }
+  // The tiles above 32 rows and the small-M kernel load A straight to LDS in
+  // 16-byte pieces: rows that don't start on 16 bytes are copied first, into
+  // the W2 output rows (no fewer bytes; written once W13 has read them).
+  const bool lds_a = smallm_mlp(a, L.routes, w8) || L.tc.bm[L.tc.n - 1] > 32;
+  uint16_t* xcopy = L.xpad ? L.xpad : lds_a && (uintptr_t)a->x % 16 ? (uint16_t*)L.route_out : nullptr;
   const uint16_t* xa = a->x;
-  if (L.xpad) {
+  if (xcopy) {
     hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)ceil_div(L.hp, 256), (unsigned)std::min<int64_t>(a->tokens, 65535)),
                        dim3(256), 0,
-                       stream, a->x, a->tokens, H, L.hp, L.xpad);
+                       stream, a->x, a->tokens, H, L.hp, xcopy);
     if ((rc = check_launch("pad_rows"))) return rc;
-    xa = L.xpad;
+    xa = xcopy;
   }
   // y columns [F, ip) feed W2's zero-padded K and must be finite zeros.
   if (I % kmul) {

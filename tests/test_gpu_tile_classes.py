@@ -85,3 +85,33 @@ def test_w8a8_weights_read_once_bit_exact(gpu, oracle_lib):
     got = H.gpu_w8a8_forward(x, ids, w, q13, s13, q2, s2, gpu)
     tok = np.array([0, 1, 74, T - 1])
     np.testing.assert_array_equal(got[tok], oracle_lib.w8a8_forward(x[tok], ids[tok], w[tok], q13, s13, q2, s2))
+
+
+@pytest.mark.parametrize("kind,T,classes", [("bf16", 70, "64"), ("w8a16", 70, "64"), ("bf16", 70, "128,192,256"),
+                                            ("w8a16", 70, "128,192,256"), ("bf16", 70, "16"), ("w8a16", 3, ""),
+                                            ("mlp", 40, ""), ("mlp", 300, "")])
+@pytest.mark.parametrize("offset", [1, 4])
+def test_rows_that_start_off_16_bytes(gpu, monkeypatch, kind, T, classes, offset):
+    """The same rows 2 or 8 bytes off a 16-byte start: bit for bit the aligned rows' result on every
+    tile (the LDS tiles load 16-byte pieces)."""
+    from fused_cpp_amd import moe
+
+    E, hd, f, k = 9, 256, 192, 2
+    g = torch.Generator(device="cuda").manual_seed(T + offset)
+    bf = lambda *s: (torch.randn(s, generator=g, device=gpu) * 0.1).to(torch.bfloat16)  # noqa: E731
+    x = bf(T, hd) * 10
+    buf = torch.zeros(T * hd + offset, dtype=torch.bfloat16, device=gpu)
+    shifted = buf[offset:].view(T, hd)
+    shifted.copy_(x)
+    assert shifted.is_contiguous() and shifted.data_ptr() % 16 == 2 * offset
+    if kind == "mlp":
+        packed = moe.prepare_shared_mlp_bf16_tiled_weights(bf(2 * f, hd), bf(hd, f))
+        call = lambda v: moe.shared_mlp_bf16_tiled(v, packed)  # noqa: E731
+    else:
+        packed = getattr(moe, f"prepare_fused_moe_{kind}_tiled_weights")(bf(E, 2 * f, hd), bf(E, hd, f))
+        ids = torch.randint(0, E, (T, k), generator=g, device=gpu)
+        w = torch.rand((T, k), generator=g, device=gpu)
+        call = lambda v: getattr(moe, f"fused_moe_{kind}_tiled")(v, packed, w, ids)  # noqa: E731
+    if classes:
+        monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
+    assert torch.equal(call(shifted).view(torch.int16), call(x).view(torch.int16))
