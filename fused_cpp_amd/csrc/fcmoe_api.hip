@@ -317,18 +317,18 @@ struct Stage {
 // small-tile classes overlap the MFMA-bound 256-row class. Streams and events
 // are per host thread and device (created on first use, default priority,
 // kept until process exit); a stage with one class launches inline.
-struct SideStreams {
-  bool ready = false;
-  hipStream_t s[kNumClasses] = {};
-  hipEvent_t fork = nullptr;
-  hipEvent_t join[kNumClasses] = {};
-};
-constexpr int kMaxDevices = 64;
 // Side streams a stage forks at most: with the caller's stream one per
 // hardware queue of a process (4). A fifth stream shares a queue with another
 // one, and its launch starts only when that one's is done: the W8A16 128-row
 // class queued behind the 192-row class (DSv3, T=4096: W13 1.36 + 1.07 ms).
 constexpr int kSides = 3;
+struct SideStreams {
+  bool ready = false;
+  hipStream_t s[kSides] = {};
+  hipEvent_t fork = nullptr;
+  hipEvent_t join[kSides] = {};
+};
+constexpr int kMaxDevices = 64;
 thread_local SideStreams t_side[kMaxDevices];
 
 int side_streams(SideStreams** out) {
@@ -339,9 +339,9 @@ int side_streams(SideStreams** out) {
   if (!ss.ready) {
     if (hipEventCreateWithFlags(&ss.fork, hipEventDisableTiming) != hipSuccess)
       return fail(FCMOE_EDEVICE, "hipEventCreate failed");
-    for (int c = 0; c < kNumClasses; ++c) {
-      if (hipStreamCreateWithFlags(&ss.s[c], hipStreamNonBlocking) != hipSuccess ||
-          hipEventCreateWithFlags(&ss.join[c], hipEventDisableTiming) != hipSuccess)
+    for (int k = 0; k < kSides; ++k) {
+      if (hipStreamCreateWithFlags(&ss.s[k], hipStreamNonBlocking) != hipSuccess ||
+          hipEventCreateWithFlags(&ss.join[k], hipEventDisableTiming) != hipSuccess)
         return fail(FCMOE_EDEVICE, "side stream creation failed");
     }
     ss.ready = true;
@@ -405,18 +405,17 @@ int run_classes(const TileClasses& tc, hipStream_t stream, F&& gemm, bool serial
   if (rc) return rc;
   if (hipEventRecord(ss->fork, stream) != hipSuccess) return fail(FCMOE_EDEVICE, "hipEventRecord failed");
   if ((rc = gemm(tc.n - 1, stream))) return rc;
-  // side stream k takes class n - 2 - k; the last one also the smaller
-  // classes, whose launches have little work
+  // side stream k takes class n - 2 - k; classes past the side streams (only
+  // FCMOE_TILE_CLASSES lists so many) follow the largest on the caller's
   const int sides = tc.n - 1 < kSides ? tc.n - 1 : kSides;
   for (int k = 0; k < sides; ++k) {
     hipStream_t s = ss->s[k];
     if ((rc = fork_wait(s, ss->fork, stream, stream))) return rc;
-    for (int c = tc.n - 2 - k; c >= 0; --c) {
-      if ((rc = gemm(c, s))) return rc;
-      if (k < sides - 1) break;
-    }
+    if ((rc = gemm(tc.n - 2 - k, s))) return rc;
     if (hipEventRecord(ss->join[k], s) != hipSuccess) return fail(FCMOE_EDEVICE, "hipEventRecord failed");
   }
+  for (int c = tc.n - 2 - sides; c >= 0; --c)
+    if ((rc = gemm(c, stream))) return rc;
   for (int k = 0; k < sides; ++k)
     if ((rc = fork_wait(stream, ss->join[k], ss->s[k], stream))) return rc;
   return FCMOE_OK;

@@ -30,7 +30,7 @@ def _ids(rng):
 
 
 @pytest.mark.parametrize("hd,f", SHAPES)
-@pytest.mark.parametrize("classes", ["16", "64", "128", "256", "128,192,256"])
+@pytest.mark.parametrize("classes", ["16", "64", "128", "256", "128,192,256", "16,32,64,128,192,256"])
 def test_w8a8_tile_edges_bit_exact(gpu, oracle_lib, monkeypatch, classes, hd, f):
     ids = _ids(np.random.default_rng(hd + f))
     x, _, w, q13, s13, q2, s2 = H.w8a8_case(hd * 3 + f, ids.shape[0], hd, f, len(ROWS), 1)
@@ -41,7 +41,8 @@ def test_w8a8_tile_edges_bit_exact(gpu, oracle_lib, monkeypatch, classes, hd, f)
 
 @pytest.mark.parametrize("hd,f", SHAPES)
 @pytest.mark.parametrize("kind,classes", [("bf16", "64"), ("bf16", "128,192,256"), ("w8a16", "64"),
-                                          ("w8a16", "128,192,256")])
+                                          ("w8a16", "128,192,256"), ("bf16", "16,32,64,128,192,256"),
+                                          ("w8a16", "16,32,64,128,192,256")])
 def test_bf16_family_tile_edges(gpu, oracle_lib, monkeypatch, kind, classes, hd, f):
     from fused_cpp_amd import moe
 
