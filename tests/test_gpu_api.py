@@ -581,14 +581,17 @@ def test_i8gemm_batched_scalar_scale_and_ties(gpu, oracle_lib):
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("classes", ["", "16,128,192,256"])
 @pytest.mark.parametrize("activation", ["silu", "swigluoai"])
-def test_bf16_prefill_every_tile_class_within_tolerance(gpu, oracle_lib, activation):
-    """Per-expert counts 3..420 reach every prefill tile class (16, 128, 192 and
-    256 rows, the last with a two-tile expert), i.e. the bf16 instantiations of
-    the register-ring kernel and of the LDS-staged prefill kernel, with biases,
-    against the fp32 reference."""
+def test_bf16_prefill_every_tile_class_within_tolerance(gpu, oracle_lib, monkeypatch, activation, classes):
+    """Per-expert counts 3..420 with biases against the fp32 reference: on the
+    64-row tiles, which the rule takes for so little work, and on every class of
+    16, 128, 192 and 256 rows (the last with a two-tile expert), i.e. the bf16
+    instantiations of the register-ring kernel and of the LDS-staged prefill
+    kernel."""
     from fused_cpp_amd import moe
 
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
     rng = np.random.default_rng(17)
     counts = [3, 20, 40, 70, 100, 150, 200, 260, 420]
     E, Hd, F = len(counts), 256, 192

@@ -94,11 +94,15 @@ def test_w8a8_one_token_decode_graph_replays(gpu):
     _replay_matches_eager(fn, make, static)
 
 
-def test_bf16_and_w8a16_forward_graph_replays(gpu):
+@pytest.mark.parametrize("T,classes", [(16, ""), (100, ""), (200, ""), (400, "128,192,256")])
+def test_bf16_and_w8a16_forward_graph_replays(gpu, monkeypatch, T, classes):
+    """The two launches of a batch of few routes (16 tokens), then route build, GEMMs and combine on
+    16-row tiles (100), 64-row tiles (200) and the forked classes of large layers (400)."""
     from fused_cpp_amd import moe
 
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
     rng = np.random.default_rng(3)
-    T, Hd, F, E, k = 16, 512, 256, 8, 2
+    Hd, F, E, k = 512, 256, 8, 2
     w13 = H.bf16_bits((rng.standard_normal((E, 2 * F, Hd)) * 0.02).astype(np.float32))
     w2 = H.bf16_bits((rng.standard_normal((E, Hd, F)) * 0.02).astype(np.float32))
     tb = lambda b: torch.from_numpy(b.view(np.int16)).to(gpu).view(torch.bfloat16)  # noqa: E731
@@ -258,16 +262,18 @@ def test_w8a8_prefill_mixed_plan_graph_replays(gpu, min_tiles):
             os.environ["FCMOE_PREFILL_MIXED_MIN_TILES"] = old
 
 
-def test_side_to_side_stream_wait_refused_under_capture(gpu):
+def test_side_to_side_stream_wait_refused_under_capture(gpu, monkeypatch):
     """The prefill fork joins side streams only through the caller's stream;
     a wait of one side stream on another's event (FCMOE_SIDE_CHAIN_WAIT=1 adds
     one) runs eagerly, bit-exact with the default fork, and is refused under
     graph capture before the forward enqueues anything (the capture then ends
-    empty and replays nothing)."""
+    empty and replays nothing). A layer of this size forks only with the
+    prefill class set forced."""
     import os
 
     from fused_cpp_amd import moe
 
+    monkeypatch.setenv("FCMOE_PREFILL_MIXED_MIN_TILES", "32")
     T, Hd, F, E, k = 2048, 1024, 512, 160, 6
     x, ids, w, q13, s13, q2, s2 = H.w8a8_case(31, T, Hd, F, E + 1, k, skew=1.2)
     ids = np.minimum(ids, E - 1)

@@ -49,7 +49,7 @@ def _case(oracle_lib, seed, T, Hd, F, E, k, w_std=0.02):
 @pytest.mark.parametrize("activation,limit", [("silu", None), ("gelu", None), ("silu", 10.0)])
 @pytest.mark.parametrize("T,Hd,F,E,k", [(16, 256, 128, 8, 2), (37, 96, 40, 5, 3), (300, 128, 64, 4, 2)])
 def test_w8a16_matches_dequantised_fp32_reference(gpu, oracle_lib, activation, limit, T, Hd, F, E, k):
-    """Unaligned H/F (zero-padded K) and multi-tile experts (32-row class at T=300)."""
+    """Unaligned H/F (zero-padded K) and multi-tile experts (about 150 rows each at T=300)."""
     from fused_cpp_amd import moe
 
     x, _, _, q13, s13, q2, s2, ids, w, deq13, deq2 = _case(oracle_lib, T * 7 + Hd, T, Hd, F, E, k)
@@ -61,16 +61,19 @@ def test_w8a16_matches_dequantised_fp32_reference(gpu, oracle_lib, activation, l
     _close(out, oracle_lib.bf16_moe_reference(x, deq13, deq2, w, ids, activation=act, round_intermediate=True))
 
 
+@pytest.mark.parametrize("classes", ["", "16,32,128,192,256"])
 @pytest.mark.parametrize("activation", ["silu", "gelu"])
 @pytest.mark.parametrize("T,Hd,F,E,k", [(200, 256, 128, 4, 2), (700, 200, 96, 4, 2), (900, 320, 160, 14, 2),
                                          (640, 256, 128, 8, 2)])
-def test_w8a16_prefill_classes(gpu, oracle_lib, activation, T, Hd, F, E, k):
+def test_w8a16_prefill_classes(gpu, oracle_lib, monkeypatch, activation, T, Hd, F, E, k, classes):
     """Prefill-sized experts on the LDS-staged W8A16 tiles: ~100 rows per
     expert (128-row class), ~350 (two 256-row tiles per expert), a mix of
     classes with unaligned H (zero-padded K) and a single-chunk W2, and ~160
-    rows per expert (192-row class)."""
+    rows per expert (192-row class); and on the 64-row tiles, which the rule
+    takes for so little work."""
     from fused_cpp_amd import moe
 
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
     x, _, _, q13, s13, q2, s2, ids, w, deq13, deq2 = _case(oracle_lib, T + 3 * Hd, T, Hd, F, E, k)
     counts = np.bincount(ids.ravel(), minlength=E)
     assert counts.max() > 32  # at least one expert beyond the direct-A tiles

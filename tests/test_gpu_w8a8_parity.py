@@ -22,7 +22,7 @@ pytestmark = pytest.mark.gpu
     "tokens,top_k,experts,shared,i64",
     [(1, 1, 1, False, True), (37, 2, 4, False, False), (64, 8, 257, True, True), (513, 6, 33, True, False),
      (4096, 8, 257, True, True),
-     # the single-workgroup path serves up to 1024 routes, the chunked one beyond
+     # one workgroup up to 1024 routes, one per 1024 beyond
      (128, 8, 9, False, True), (114, 8, 1024, True, False), (103, 10, 1000, False, True)],
 )
 def test_route_build_matches_oracle(gpu, oracle_lib, tokens, top_k, experts, shared, i64):
@@ -166,7 +166,19 @@ def test_w8a8_forward_bit_exact_dsv3_hidden(gpu, oracle_lib):
     _check_w8a8(gpu, oracle_lib, case, shared=True, scale=2.5)
 
 
-def test_w8a8_forward_bit_exact_skewed_prefill(gpu, oracle_lib):
+# The rule's own class set (a layer of so little work takes 64-row tiles), and the four classes and
+# launch plans of the large W8A8 layers.
+CLASS_SETS = ["", "16,128,192,256"]
+
+
+@pytest.fixture(params=CLASS_SETS, ids=["rule", "prefill"])
+def class_set(request, monkeypatch):
+    if request.param:
+        monkeypatch.setenv("FCMOE_TILE_CLASSES", request.param)
+    return request.param
+
+
+def test_w8a8_forward_bit_exact_skewed_prefill(gpu, oracle_lib, class_set):
     """Zipf-skewed routing over 64 experts: every tile class, empty experts."""
     case = H.w8a8_case(9, 1024, 256, 128, 65, 8, skew=1.2)
     _check_w8a8(gpu, oracle_lib, case, shared=True, scale=2.5)
@@ -177,7 +189,7 @@ def test_w8a8_forward_bit_exact_skewed_prefill(gpu, oracle_lib):
     (600, 208, 80, 9, 4, 1.2),       # ragged K on every tile class, the LDS kernel included
     (333, 1040, 272, 17, 6, 1.1),    # K = 1040 / 272: padded tail chunk after full ones
 ])
-def test_w8a8_forward_bit_exact_ragged_dims(gpu, oracle_lib, tokens, hidden, inter, experts, top_k, skew):
+def test_w8a8_forward_bit_exact_ragged_dims(gpu, oracle_lib, class_set, tokens, hidden, inter, experts, top_k, skew):
     """H and F multiples of 16 but not of 64 (the reference's W8A8 domain,
     csrc/moe/arm/i8mm_w8a8/kernels.cpp:485-570): the packed K chunks and the
     quantised activation rows carry zero padding that must not change a bit."""
@@ -193,7 +205,7 @@ def test_w8a8_forward_repeat_bitwise(gpu, oracle_lib):
     np.testing.assert_array_equal(a, b)
 
 
-def test_w8a8_forward_bit_exact_odd_chunk_counts(gpu, oracle_lib):
+def test_w8a8_forward_bit_exact_odd_chunk_counts(gpu, oracle_lib, class_set):
     """K = 1040 / 272 (17 / 5 chunks of 64 bytes): the LDS-staged kernel loads
     A two chunks at a time, so its last A stage lies half past K; the 600- and
     256-row experts run the 256-row tiles (W13 on 4-wave workgroups, W2 and
@@ -215,10 +227,9 @@ def test_w8a8_forward_bit_exact_odd_chunk_counts(gpu, oracle_lib):
 
 @pytest.mark.parametrize("tokens", [128, 129])
 def test_w8a8_forward_bit_exact_route_path_boundary(gpu, oracle_lib, tokens):
-    """1024 routes (128 tokens x top-8) is the largest routing the single-
-    workgroup route kernel takes, and there the token rows are quantised in
-    the same launch (32 groups of 4 rows); 129 tokens (1032 routes) take the
-    count / scan / scatter kernels and the separate row quantisation."""
+    """1024 routes (128 tokens x top-8) fill one routing workgroup of the route
+    launch, beside 32 of 4 quantised token rows each; 129 tokens (1032 routes)
+    take two, beside 33 whose last has one row."""
     case = H.w8a8_case(900 + tokens, tokens, 512, 256, 16, 8)
     _check_w8a8(gpu, oracle_lib, case, shared=False)
 

@@ -13,14 +13,16 @@ from tests.helpers import gpu_w8a8_forward, pack_gpu, w8a8_case
 pytestmark = pytest.mark.gpu
 
 
-def test_noalloc_matches_workspace_forward_on_two_calls(gpu):
+def test_noalloc_matches_workspace_forward_on_two_calls(gpu, monkeypatch):
     H, I, E, k = 1024, 512, 16, 8
     x, ids, w, q13, s13, q2, s2 = w8a8_case(4242, 96, H, I, E + 1, k)
     ids = np.minimum(ids, E - 1)  # routed ids stay below the shared slot
     packed = (pack_gpu(q13, 2, gpu), pack_gpu(q2, 1, gpu))
-    # 96 tokens: several prefill tile classes (run in order on one stream);
-    # 5 tokens: the single decode class; 1 token: the decode head and tail launches.
-    for tokens in (96, 5, 1):
+    # 96 tokens: several prefill tile classes (run in order on one stream), then
+    # the rule's 64-row tiles; 20 tokens: the 16-row tiles; 5 and 1 tokens: the
+    # decode head and tail launches.
+    for tokens, classes in ((96, "16,128,192,256"), (96, ""), (20, ""), (5, ""), (1, "")):
+        monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
         print(f"[noalloc] tokens={tokens} H={H} I={I} E={E}+1 top-{k}", flush=True)
         args = (x[:tokens], ids[:tokens], w[:tokens], q13, s13, q2, s2, gpu)
         kw = dict(shared_id=E, scale=2.5, packed=packed)
