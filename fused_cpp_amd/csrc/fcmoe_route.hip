@@ -8,7 +8,8 @@
 // the appended shared expert with weight 1.0 and the routed weights are scaled
 // by routed_scaling_factor (src/fused_cpp/moe/bf16_tiled.py:1007-1013).
 //
-// One launch up to kOneLaunchRoutes routes (route_all_kernel): every
+// One launch for tens of thousands of routes (route_all_kernel, up to
+// one_route_launch's line): every
 // 1024-route workgroup builds the whole histogram over experts from the ids
 // itself, taking a copy before its own routes, so that no workgroup waits for
 // another; workgroup 0 also writes the counts, offsets and tile lists (the
@@ -333,7 +334,22 @@ struct RouteOut {
 // from wcnt. DSv3 W8A8, route + row quantisation, MI355X: T=333 27 -> 8.5 us,
 // T=4096 47 -> 36, T=8192 E=384 73 -> 65; 64 tokens 11.8 -> 6.4 (there
 // one workgroup ranked each route against all earlier ones).
-constexpr int kOneLaunchRoutes = 1 << 18;
+//
+// Where it ends: it saves about 10 us (two launches and their waits), and a
+// route costs it some 0.31 ns more than the three launches, whose scan in turn
+// grows with experts x routes (0.5 ps a route and expert). us of one launch
+// against three, uniform ids, with the same result copies: 8 experts 32768
+// routes 25.9 / 27.6 (Zipf 31.6 / 29.9), 65536 37.2 / 29.2, 262144 103 / 41; 65
+// experts 32768 26.4 / 28.4, 65536 37.8 / 30.0; 257 experts 32768 26.0 / 30.8,
+// 65536 37.0 / 35.1, 262144 103 / 75; 385 experts 65536 37.1 / 38.8, 98304 49.0
+// / 47.7, 262144 104 / 93; 1024 experts 65536 36.1 / 54.2, 262144 96.8 / 148.
+constexpr int kOneLaunchRoutes = 1 << 18;  // the largest measured
+
+bool one_route_launch(int64_t routes, int64_t experts) {
+  const int64_t ps = 310 - experts / 2;  // what a route costs the one launch more
+  return routes <= kOneLaunchRoutes && routes * ps <= 10000000;
+}
+
 constexpr int kRouteWaves = kScanThreads / kWave;
 constexpr int kIdBatch = 8;  // ids a thread has in flight
 
@@ -570,7 +586,7 @@ int route_launch(const void* ids, int ids_is_i64, const float* topk_w, int64_t t
   const int64_t chunks = ceil_div(routes, kRouteChunk);
   int32_t* invalid = invalid_out ? invalid_out : rb.invalid;
   const ClassArgs ca = class_args(tc);
-  if (routes <= kOneLaunchRoutes) {
+  if (one_route_launch(routes, experts)) {
     const RouteOut o{rb.counts,    rb.offsets,   rb.tiles,        rb.tile_count, rb.sorted_routes,
                      rb.row_token, rb.route_pos, rb.route_weight, invalid,      rb.queues};
     const int wgs = (int)ceil_div(routes, kScanThreads);

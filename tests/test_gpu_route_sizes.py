@@ -17,7 +17,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("tokens,k,experts,shared", [
     (1, 1, 1, False), (63, 1, 5, False), (341, 3, 1024, False), (128, 8, 257, True), (1024, 1, 2, False),
-    (1025, 1, 1000, False), (114, 8, 257, True), (5000, 6, 21, True), (32768, 8, 384, False), (32769, 8, 129, False)])
+    (1025, 1, 1000, False), (114, 8, 257, True), (5000, 6, 21, True), (32768, 8, 384, False), (32769, 8, 129, False),
+    # both sides of the line that depends on the experts, and of the line for all
+    (16339, 2, 8, False), (16340, 2, 8, False), (9416, 8, 385, True), (9417, 8, 385, True), (32768, 8, 1024, False),
+    (32769, 8, 1024, False)])
 def test_route_build_sizes(gpu, tokens, k, experts, shared):
     rng = np.random.default_rng(tokens + k)
     valid = experts - 1 if shared else experts
