@@ -57,14 +57,25 @@ int class_slot(int bm) {
 //     while the layer's operations are few: what a larger tile would save in
 //     weight re-reads is less than what its longer K walk on a few dozen
 //     workgroups costs. TP W8A8 T=200 180 -> 55, T=1000 244 -> 146; BF16 T=200
-//     253 -> 94, T=1000 322 -> 225; W8A16 T=400 246 -> 88 (the larger figure:
-//     128-row and larger class launches on forked streams). The operations bound: TP BF16 T=1000
-//     (88 GFLOP) 225 against 257 on 128 rows, T=2047 (180) 422 against 319 (293
-//     with the staged epilogue);
-//     one BF16 expert at 1000 rows (88) 246 against 288, at 2000 (180) 478
-//     against 332; 8 DSv3 W8A8 experts at T=256 (203 GOP) 298 against 181.
+//     253 -> 94; W8A16 T=400 246 -> 88 (the larger figure: 128-row and larger
+//     class launches on forked streams). The operations bound, 64 rows against
+//     128 (19 shapes, uniform and Zipf): BF16 and W8A8 cross between 60 and 90
+//     GOP (8 experts of 1536 x 4096 BF16 T=600 / 800 / 1200 / 1600, 45 / 60 /
+//     91 / 121 GOP, 1.17x faster / 0.94 / 0.80 / 0.67; 32 of 2048 x 1024 W8A8
+//     T=1600, 81 GOP, 0.87), and none of the 86 points of 8 and more experts
+//     from 80 on is 2% better on 64 rows; one or two experts, whose larger tiles
+//     are few, cross at 91 (one BF16 expert of DSv3 at 1000 rows, 88 GOP, 1.12,
+//     at 1100, 97, 0.97; one W8A8 expert at 1000 1.12, at 1100 1.00). W8A16
+//     crosses at 110 (120-190 GOP 0.85 to 1.17). And within r = 48 W8A8 does above
+//     120 GOP (160 experts of 1536 x 5120 top-6 + 1 T=800, 264 GOP, r = 35, 908
+//     against 730; Zipf 1001 against 808).
 //   * 128-row tiles above; 256-row ones when experts hold many tiles of either
-//     (r > 1000: TP W8A8 T=4000 363 against 401, BF16 569 against 599).
+//     (r > 1000: TP W8A8 T=4000 363 against 401, BF16 569 against 599). From 2
+//     GB of weights {128, 192, 256} where most experts are one 192- or 256-row
+//     tile (r 128 to 256): 64 experts of 2048 x 7168 top-8 + 1 T=1200 W8A8 1070
+//     -> 828, W8A16 1582 -> 1297; smaller layers lose to the fork (BF16 of 1-2 GB
+//     0.97 in the mean, Zipf-routed 0.88), and so does a short W2 (BF16 DSv3
+//     with F = 256 T=4096 Zipf 1086 against 1218).
 //   * Layers of more than kBigWeights: 64 rows up to r = 10 (W8A8; T=256 1871 ->
 //     1808), 16 (BF16; 128 experts T=128 1840 -> 1751) or 24 (W8A16; T=512 2119
 //     -> 1923); one 128-row class up to r = 48 (W8A8 T=1024 2078 -> 2030,
@@ -73,6 +84,7 @@ int class_slot(int bm) {
 //     -> 4051). W8A8 above r = 96 keeps the launch plans of run_w8a8_stage.
 enum Family { kW8A8, kBf16, kW8A16 };
 constexpr int64_t kBigWeights = 4ll << 30;
+constexpr int64_t kForkWeights = 2ll << 30;
 // Layers of more weight bytes than this do not stay in the Infinity Cache (256
 // MB): 64-row tiles that read an expert once (r <= 48) load them nontemporal
 // (DSv3 T=64 1623 -> 1510, one 8-expert layer of 132 MB 50 -> 55).
@@ -144,7 +156,10 @@ TileClasses select_classes(const MoeShape& m, bool lds = true) {
     return set({128, 192, 256});
   }
   const int64_t gop = 6 * m.routes * m.hidden * m.inter / 1000000000;
-  if (m.few_rows(48) || gop <= (m.family == kW8A8 ? 90 : m.family == kBf16 ? 120 : 110)) return set({64});
+  if (m.few_rows(48) && (m.family != kW8A8 || gop <= 120)) return set({64});
+  if (gop < (m.family == kW8A16 ? 111 : m.experts < 8 ? 91 : 80)) return set({64});
+  if (m.weight_bytes() > kForkWeights && m.inter * m.elem() > 512 && m.few_rows(256) && !m.few_rows(128))
+    return set({128, 192, 256});
   return m.few_rows(1000) ? set({128}) : set({256});
 }
 

@@ -116,3 +116,55 @@ def test_rows_that_start_off_16_bytes(gpu, monkeypatch, kind, T, classes, offset
     if classes:
         monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
     assert torch.equal(call(shifted).view(torch.int16), call(x).view(torch.int16))
+
+
+@pytest.mark.parametrize("family,T,hd,f,experts,k,shared,classes", [
+    # work from 80 GOP leaves the 64-row tiles (64 against 128 rows, us: 331 / 222, 536 / 334, 152 / 132), of few
+    # experts from 91 (284 / 275), W8A16's from 111
+    ("bf16", 1600, 4096, 1536, 8, 2, False, "128"), ("bf16", 600, 2880, 2880, 32, 4, False, "128"),
+    ("bf16", 1100, 7168, 2048, 2, 1, False, "128"), ("w8a8", 1600, 1024, 2048, 32, 4, False, "128"),
+    ("bf16", 800, 4096, 1536, 8, 2, False, "64"), ("w8a8", 1000, 7168, 2048, 1, 1, False, "64"),
+    ("bf16", 1000, 7168, 2048, 1, 1, False, "64"),
+    ("w8a16", 1200, 4096, 1536, 8, 2, False, "64"),
+    # at most 48 rows per expert: W8A8's from 120 GOP (908 / 730), W8A16's not
+    ("w8a8", 800, 5120, 1536, 160, 6, True, "128"), ("w8a8", 400, 5120, 1536, 160, 6, True, "128"),
+    ("w8a8", 350, 5120, 1536, 160, 6, True, "64"), ("w8a16", 300, 7168, 2048, 64, 8, True, "64"),
+    # over 2 GiB of weights and 128 to 256 rows per expert: three classes (128 rows against them: 1070 / 828)
+    ("w8a8", 1200, 7168, 2048, 64, 8, True, "128,192,256"), ("w8a16", 1600, 7168, 2048, 64, 8, True, "128,192,256"),
+    ("w8a8", 900, 7168, 2048, 64, 8, True, "128"), ("w8a8", 2400, 7168, 2048, 64, 8, True, "128"),
+    ("w8a8", 2400, 4096, 1536, 64, 4, True, "128"), ("bf16", 4096, 7168, 256, 256, 8, True, "128")])
+def test_tile_class_rule(gpu, family, T, hd, f, experts, k, shared, classes):
+    """The class set on both sides of the rule's lines, from the stages that ran (weights of zeros)."""
+    import ctypes
+
+    from fused_cpp_amd import cabi
+
+    L = cabi.lib()
+    size = 2 if family == "bf16" else 1
+    total = experts + shared
+    keep = {
+        "x": torch.zeros((T, hd), dtype=torch.bfloat16, device=gpu),
+        "topk_ids": torch.randint(0, experts, (T, k), device=gpu),
+        "topk_weights": torch.ones((T, k), device=gpu),
+        "w13": torch.zeros(total * L.fcmoe_packed_expert_bytes(size, 2 * f, hd, 2), dtype=torch.uint8, device=gpu),
+        "w2": torch.zeros(total * L.fcmoe_packed_expert_bytes(size, hd, f, 1), dtype=torch.uint8, device=gpu),
+        "out": torch.ones((T, hd), dtype=torch.bfloat16, device=gpu)}
+    if size == 1:
+        keep["w13_scale"], keep["w2_scale"] = torch.ones((total, 2 * f), device=gpu), torch.ones((total, hd), device=gpu)
+    a = cabi.MoeArgs()
+    a.tokens, a.hidden, a.inter, a.top_k, a.ids_is_i64, a.routed_scaling = T, hd, f, k, 1, 1.0
+    a.experts, a.valid_experts, a.shared_expert_id = total, experts, experts if shared else -1
+    a.activation = cabi.FCMOE_ACT_SILU_CLAMP10
+    a.workspace_bytes = getattr(L, f"fcmoe_{family}_workspace_bytes")(ctypes.byref(a))
+    keep["workspace"] = torch.empty(a.workspace_bytes, dtype=torch.uint8, device=gpu)
+    for name, t in keep.items():
+        setattr(a, name, t.data_ptr())
+    cabi.stage_timing_read()
+    cabi.stage_timing_enable(True)
+    try:
+        cabi.check(getattr(L, f"fcmoe_{family}_forward")(ctypes.byref(a), cabi.stream_handle()), "forward")
+        ran = cabi.stage_timing_read()
+    finally:
+        cabi.stage_timing_enable(False)
+    assert {s for s in ran if "bm" in s} == {f"{w}_bm{c}" for w in ("w13", "w2") for c in classes.split(",")}
+    assert not keep["out"].any()
