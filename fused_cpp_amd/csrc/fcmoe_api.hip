@@ -48,7 +48,10 @@ int class_slot(int bm) {
 //     1510 on 64-row tiles, T=128 (r = 4.5) 1706 against 1704. BF16 and W8A16
 //     move to 64 rows at r = 2 (128 experts, r = 2.2: BF16 1537 -> 1508, DSv3
 //     W8A16 T=64 1508 -> 1490; 384 experts BF16 T=70, r = 1.6, 3991 against
-//     4142), and so does a layer whose W2 is a short K over
+//     4142), BF16 layers of at most 64 experts at 3 (40 of 1024 x 2048 top-4
+//     T=24 91 against 98, 49 of 768 x 1024 top-6 + 1 T=16 54 against 60) and of
+//     fewer than 32 at 5 (16 of 2048 x 6144 top-2 + 1 T=24 211 against 240, TP
+//     T=12 62 against 64), where W8A16 gains up to 1.3x on 64; and so does a layer whose W2 is a short K over
 //     many experts, where the 16-row kernel's workgroups are all set-up (DSv3
 //     with F = 256 T=16 161 -> 114, T=100 389 -> 278; the few workgroups of TP
 //     at T=2 stay, 30 against 37). Layers that fit an L2 stay up to r = 32
@@ -145,7 +148,8 @@ TileClasses select_classes(const MoeShape& m, bool lds = true) {
   // 16-row tiles of a short W2 (at most 8 chunks of K) over many experts
   const bool short_w2 = m.inter * m.elem() <= 512 && m.routes > 64 && m.weight_bytes() > kCachedWeights;
   const bool in_l2 = m.weight_bytes() <= 64ll << 20;
-  const bool one_row = m.few_rows(m.family == kW8A8 ? 4 : 2);
+  const bool few_experts = m.family == kBf16 && !big;
+  const bool one_row = m.few_rows(m.family == kW8A8 ? 4 : few_experts && m.experts < 32 ? 5 : few_experts && m.experts <= 64 ? 3 : 2);
   if (tiny || (one_row && !short_w2) || (in_l2 && m.few_rows(32))) return set({16});
   const char* forced = getenv("FCMOE_PREFILL_MIXED_MIN_TILES");
   if (m.family == kW8A8 && ((big && !m.few_rows(96)) || (forced && forced[0])))

@@ -132,7 +132,12 @@ def test_rows_that_start_off_16_bytes(gpu, monkeypatch, kind, T, classes, offset
     # over 2 GiB of weights and 128 to 256 rows per expert: three classes (128 rows against them: 1070 / 828)
     ("w8a8", 1200, 7168, 2048, 64, 8, True, "128,192,256"), ("w8a16", 1600, 7168, 2048, 64, 8, True, "128,192,256"),
     ("w8a8", 900, 7168, 2048, 64, 8, True, "128"), ("w8a8", 2400, 7168, 2048, 64, 8, True, "128"),
-    ("w8a8", 2400, 4096, 1536, 64, 4, True, "128"), ("bf16", 4096, 7168, 256, 256, 8, True, "128")])
+    ("w8a8", 2400, 4096, 1536, 64, 4, True, "128"), ("bf16", 4096, 7168, 256, 256, 8, True, "128"),
+    # 16-row tiles of BF16 layers of few experts (us on 16 / 64 rows: 91 / 98, 54 / 60, 211 / 240)
+    ("bf16", 24, 2048, 1024, 40, 4, False, "16"), ("bf16", 16, 1024, 768, 48, 6, True, "16"),
+    ("bf16", 24, 6144, 2048, 16, 2, True, "16"), ("bf16", 48, 2048, 1024, 40, 4, False, "64"),
+    ("bf16", 48, 6144, 2048, 16, 2, True, "64"), ("bf16", 40, 2048, 768, 128, 8, False, "64"),
+    ("w8a16", 24, 6144, 2048, 16, 2, True, "64")])
 def test_tile_class_rule(gpu, family, T, hd, f, experts, k, shared, classes):
     """The class set on both sides of the rule's lines, from the stages that ran (weights of zeros)."""
     import ctypes
