@@ -608,7 +608,13 @@ bool part_enabled() {
 // launches are most of its time gains (us: 8 experts of 512 x 1024 top-2 W8A8 T=8
 // 26 -> 16, BF16 T=32 22 -> 17; TP rank of H 4096, F 512, top-6 BF16 T=1 30 -> 21,
 // W8A16 T=2 44 -> 22, W8A8 T=4 33 -> 27), and one that is bound by its
-// weights loses (DSv3 W8A8 T=2 120 -> 124 us, T=4 215 -> 227).
+// weights loses (DSv3 W8A8 T=2 120 -> 124 us, T=4 215 -> 227). Over 16 shapes of
+// 1 to 64 experts and the three types, weights not cached, the other launches'
+// time over the two launches': up to 192 MB of streams 1.0 to 2.4 (one W8A8
+// shape, 128 x 8192 T=16, 0.96), 216-288 MB 0.97 to 1.7, 336-384 MB 0.75 to 1.9,
+// from 576 MB 0.4 to 1.3. Few experts that many routes share are no worse: 8 of
+// 512 x 1024 BF16 T=32 (192 MB) 25 -> 21 us, 2 of 512 x 2048 W8A16 T=32 40 ->
+// 30, one of 2048 x 7168 W8A16 T=4 66 -> 31.
 // FCMOE_DECODE_TAIL_MAX_T, when set, is the W8A8 batches' rule instead: at most
 // this many tokens (0: none) take the tail, and one-token ones the head.
 constexpr int64_t kSmallBatchBytes = 200ll << 20;
