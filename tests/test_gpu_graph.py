@@ -43,9 +43,12 @@ def _replay_matches_eager(fn, make_inputs, static_inputs, replays=3):
         assert torch.isfinite(noise)
 
 
-def test_w8a8_forward_graph_replays(gpu):
+@pytest.mark.parametrize("classes", ["", "64", "128,192,256"])
+def test_w8a8_forward_graph_replays(gpu, monkeypatch, classes):
+    """One launch per stage on 16- and 64-row tiles, and the forked classes of layers of 2 to 4 GB."""
     from fused_cpp_amd import moe
 
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
     case = H.w8a8_case(21, 48, 1024, 512, 17, 4)
     x, ids, w, q13, s13, q2, s2 = case
     t = torch.from_numpy
@@ -94,10 +97,11 @@ def test_w8a8_one_token_decode_graph_replays(gpu):
     _replay_matches_eager(fn, make, static)
 
 
-@pytest.mark.parametrize("T,classes", [(16, ""), (100, ""), (200, ""), (400, "128,192,256")])
+@pytest.mark.parametrize("T,classes", [(16, ""), (100, ""), (200, ""), (400, "128,192,256"), (20000, "")])
 def test_bf16_and_w8a16_forward_graph_replays(gpu, monkeypatch, T, classes):
     """The two launches of a batch of few routes (16 tokens), then route build, GEMMs and combine on
-    16-row tiles (100), 64-row tiles (200) and the forked classes of large layers (400)."""
+    16-row tiles (100), 64-row tiles (200) and the forked classes of large layers (400); the route build
+    of 40000 routes in three launches (20000)."""
     from fused_cpp_amd import moe
 
     monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
