@@ -487,16 +487,17 @@ def test_i8gemm_small_m_split_k_bit_exact(gpu, oracle_lib, m, k, n, bias, out_dt
         np.testing.assert_array_equal(got.numpy().view(np.uint32), ref.view(np.uint32))
 
 
-@pytest.mark.parametrize("kind", ["bf16", "w8a16"])
-def test_forward_activation_rows_beyond_2gib(gpu, oracle_lib, kind):
+@pytest.mark.parametrize("kind,classes", [("bf16", ""), ("bf16", "64"), ("bf16", "128,192,256"), ("w8a16", "")])
+def test_forward_activation_rows_beyond_2gib(gpu, oracle_lib, monkeypatch, kind, classes):
     """Maximum sizes: 150000 x 7168 bf16 token rows (2.15 GB) exceed the 2 GiB a
-    32-bit buffer offset reaches. BF16's W13 then runs its 128-256-row tiles on
-    the 64-bit-addressed register kernel, and W8A16 keeps to its 16/32-row
-    classes. Tokens before, across and after the boundary are checked against
+    32-bit buffer offset reaches. BF16's W13 then runs its tiles (of 256 rows by
+    the rule; 64 rows, and all that a fork has) on the 64-bit-addressed register
+    kernel, and W8A16 keeps to its 16/32-row classes. Tokens before, across and after the boundary are checked against
     the fp32 reference (tokens are independent, so the reference only needs
     the sampled ones), within max-abs 2e-2 and cosine 0.9999."""
     from fused_cpp_amd import moe
 
+    monkeypatch.setenv("FCMOE_TILE_CLASSES", classes)
     T, Hd, F, E = 150000, 7168, 64, 2
     g = torch.Generator(device=gpu)
     g.manual_seed(5)
