@@ -45,17 +45,20 @@ int class_slot(int bm) {
 // experts, top-2 ("8x512"):
 //   * 16-row tiles (register-ring kernel, weights streamed once per 16 rows)
 //     while experts see a row or two: DSv3 W8A8 T=64 (r = 2.2) 1490 against
-//     1510 on 64-row tiles, T=128 (r = 4.5) 1706 against 1704. BF16 and W8A16
-//     move to 64 rows at r = 2 (128 experts, r = 2.2: BF16 1537 -> 1508, DSv3
-//     W8A16 T=64 1508 -> 1490; 384 experts BF16 T=70, r = 1.6, 3991 against
-//     4142), BF16 layers of at most 64 experts at 3 (40 of 1024 x 2048 top-4
-//     T=24 91 against 98, 49 of 768 x 1024 top-6 + 1 T=16 54 against 60) and of
-//     fewer than 32 at 5 (16 of 2048 x 6144 top-2 + 1 T=24 211 against 240, TP
-//     T=12 62 against 64), where W8A16 gains up to 1.3x on 64; and so does a layer whose W2 is a short K over
-//     many experts, where the 16-row kernel's workgroups are all set-up (DSv3
-//     with F = 256 T=16 161 -> 114, T=100 389 -> 278; the few workgroups of TP
-//     at T=2 stay, 30 against 37). Layers that fit an L2 stay up to r = 32
-//     (8x512 T=100 27 against 31).
+//     1510 on 64-row tiles. From r = 4 to 10 the two are level to 7% apart under
+//     uniform routing, the 16-row ones ahead (DSv3 W8A8 T=150 1728 / 1767-1846,
+//     128 experts of 3072 x 7168 T=72 1274 / 1266), and the 64-row ones 8 to 25%
+//     ahead under Zipf routing (1522 / 1354, 1052 / 926). BF16 and W8A16 move to
+//     64 rows at r = 2 (128 experts, r = 2.2: BF16 1537 -> 1508, DSv3 W8A16 T=64
+//     1508 -> 1490; 384 experts BF16 T=70, r = 1.6, 3991 against 4142), BF16
+//     layers of at most 64 experts at 3 (40 of 1024 x 2048 top-4 T=24 91 against
+//     98, 49 of 768 x 1024 top-6 + 1 T=16 54 against 60) and of fewer than 32 at
+//     5 (16 of 2048 x 6144 top-2 + 1 T=24 211 against 240, TP T=12 62 against
+//     64), where W8A16 gains up to 1.3x on 64; and so does a layer whose W2 is a
+//     short K over many experts, where the 16-row kernel's workgroups are all
+//     set-up (DSv3 with F = 256 T=16 161 -> 114, T=100 389 -> 278; the few
+//     workgroups of TP at T=2 stay, 30 against 37). Layers that fit an L2 stay
+//     up to r = 32 (8x512 T=100 27 against 31).
 //   * 64-row tiles (fcmoe_gemm_mid.hip) from there to r = 48, and beyond it
 //     while the layer's operations are few: what a larger tile would save in
 //     weight re-reads is less than what its longer K walk on a few dozen
