@@ -151,8 +151,9 @@ TileClasses select_classes(const MoeShape& m, bool lds = true) {
   // 16-row tiles of a short W2 (at most 8 chunks of K) over many experts
   const bool short_w2 = m.inter * m.elem() <= 512 && m.routes > 64 && m.weight_bytes() > kCachedWeights;
   const bool in_l2 = m.weight_bytes() <= 64ll << 20;
-  const bool few_experts = m.family == kBf16 && !big;
-  const bool one_row = m.few_rows(m.family == kW8A8 ? 4 : few_experts && m.experts < 32 ? 5 : few_experts && m.experts <= 64 ? 3 : 2);
+  int64_t rows16 = m.family == kW8A8 ? 4 : 2;
+  if (m.family == kBf16 && !big) rows16 = m.experts < 32 ? 5 : m.experts <= 64 ? 3 : 2;
+  const bool one_row = m.few_rows(rows16);
   if (tiny || (one_row && !short_w2) || (in_l2 && m.few_rows(32))) return set({16});
   const char* forced = getenv("FCMOE_PREFILL_MIXED_MIN_TILES");
   if (m.family == kW8A8 && ((big && !m.few_rows(96)) || (forced && forced[0])))
